@@ -242,147 +242,270 @@ __global__ __launch_bounds__(NTHR, 2) void attn_fwd_mfma(AttnArgs a) {
   }
 }
 
-// sum / max over the 16 lanes of a row (DPP row rotations, no LDS): every
-// lane of the row gets the result
-template <int R>
-__device__ inline float row_ror(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + R, 0xf, 0xf, false));
-}
-__device__ inline float row_sum16(float v) {
-  v += row_ror<8>(v);
-  v += row_ror<4>(v);
-  v += row_ror<2>(v);
-  return v + row_ror<1>(v);
-}
-__device__ inline float row_max16(float v) {
-  v = fmaxf(v, row_ror<8>(v));
-  v = fmaxf(v, row_ror<4>(v));
-  v = fmaxf(v, row_ror<2>(v));
-  return fmaxf(v, row_ror<1>(v));
+// fp32 path (any F32 request). v_mfma_f32_16x16x4_f32 forms both products
+// in fp32 (fp32 operands, products and sums: the HTile recurrence with no
+// rounding of P, the input type being fp32).
+//
+// A work-group takes 16 * NQ query rows, and its NW waves share out the keys:
+// wave w runs the online softmax (m, l, O) over the 16-key blocks w, w + NW,
+// .. for all of those rows, and the NW states of a row are merged at the end
+// through LDS in the exp2 domain (M = max m_w, l = sum 2^(m_w - M) l_w, the
+// same for O). As in the 16-bit kernels each wave forms the transposed products
+//   S^T = K . Q^T    O^T = V^T . P^T
+// so lane (i = lane % 16, g = lane / 16) holds query i's scores of keys 4 g + r
+// (r = 0..3) of the block, which is the B operand of P.V as it stands. No key
+// or value is read by two waves, so K and V go straight from memory to the A
+// operand registers, 16 bytes a lane: the k index of a product may be any
+// order that both operands share, and a row index any order the result is
+// read back in, so a lane takes four neighbouring head_dim elements of its
+// key (K), and four neighbouring head_dim rows of V^T. K of the next block is
+// loaded while this one's softmax and P.V run, V at the top of its own block.
+//
+// Bound: fp32 MFMA, D/2 instructions of 32 cycles per 16 keys and 16 rows;
+// they run on the vector ALU's own multipliers, so the softmax does not hide
+// behind them. The NQ column blocks share every K and V load. Measured (GPU
+// time, against a vector-ALU kernel that held one key's whole dot product
+// in a lane): B2 H12 S1500 D64 causal 361 -> 81 us (85 TFLOP/s; a large fp32
+// GEMM reaches 154 on this card), B2 H16 S1024 D128 1434 -> 162 us (106
+// TFLOP/s), B1 H1 S128 D64 10.3 -> 4.9 us (three quarters of it launch
+// latency).
+constexpr int F32_KB = 16;  // keys per block and wave
+// The split of the work by the number of 32-row blocks of the launch. Below
+// the line the GPU is short of work-groups and a wave's serial key loop sets
+// the time, so 16-row work-groups cut the keys eight ways; above it the
+// matrix units are full and 32-row work-groups of 4 waves read K and V half
+// as often. Measured at D = 64 (us, 16-row / 32-row): no mask 128 blocks
+// 15.4 / 22.8, 256 blocks 28.3 / 24.8; causal, where the late blocks hold
+// most of the work, 256 blocks 21.1 / 22.9, 512 blocks 21.5 / 19.6 (S 512)
+// and 32.1 / 33.3 (S 1024). D = 32 and 128 cross at the same counts.
+constexpr int64_t F32_FILL = 256, F32_FILL_CAUSAL = 512;
+
+template <int N>
+struct F32Vec;
+template <>
+struct F32Vec<4> { typedef f32x4 type; };
+template <>
+struct F32Vec<2> { typedef f32x2 type; };
+
+// N consecutive floats; VEC: the address is a multiple of 4 N bytes
+template <int N, bool VEC>
+__device__ inline typename F32Vec<N>::type load_f32(const float *p) {
+  typedef typename F32Vec<N>::type V;
+  if constexpr (VEC) return *(const V *)p;
+  V v;
+#pragma unroll
+  for (int e = 0; e < N; ++e) v[e] = p[e];
+  return v;
 }
 
-// fp32 path (config 1 and any F32 request): a 256-thread work-group per 16
-// query rows, 16 lanes per row. K/V blocks of 64 keys are staged in LDS;
-// lane k of a row takes keys k, k + 16, k + 32, k + 48 of each block and
-// keeps its own online-softmax state (m, l, acc) over them, the HTile
-// recurrence with no rounding of P (the input type is fp32). The 16 states
-// of a row are merged at the end in the exp2 domain, M = max m_k,
-// l = sum 2^(m_k - M) l_k, acc = sum 2^(m_k - M) acc_k (the flash-decoding
-// combine), so a short sequence still spreads over many waves.
-constexpr int F32_BM = 16;   // query rows per work-group
-constexpr int F32_KS = 16;   // lanes per row, each taking every 16th key
-constexpr int F32_NT = F32_BM * F32_KS;
+// VEC: 16-byte loads and stores (every base and stride a multiple of 16
+// bytes); otherwise one element each
+template <int D, bool CAUSAL, int NQ, int NW, bool VEC>
+__global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
+  constexpr int NM = D / 16;             // 16-wide head_dim blocks
+  constexpr int VW = NM < 4 ? NM : 4;    // head_dim elements per V load
+  constexpr int VL = NM / VW;            // V loads per key
+  constexpr int ROWS = 16 * NQ;
+  constexpr int OP = D + 4;              // row pitch of the merge buffer
+  typedef typename F32Vec<VW>::type VV;
+  __shared__ __attribute__((aligned(16))) float mo[NW][ROWS][OP];
+  __shared__ float mm[NW][ROWS], ml[NW][ROWS];
 
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(F32_NT) void attn_fwd_f32(AttnArgs a) {
-  // rows padded by 4 floats: the 16 lanes of a row read 16 different keys
-  // at one head_dim offset, spread over the banks
-  constexpr int DP = D + 4;
-  __shared__ __attribute__((aligned(16))) float Ks[BN][DP];
-  __shared__ __attribute__((aligned(16))) float Vs[BN][DP];
-  const int t = threadIdx.x;
-  const int rl = t / F32_KS, kl = t % F32_KS;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
   const int id = blockIdx.x;
-  const int qb = id / a.BH, bh = id % a.BH;
+  // heaviest causal query blocks first
+  const int qb = CAUSAL ? a.nqb - 1 - id / a.BH : id / a.BH;
+  const int bh = id % a.BH;
   const int b = bh / a.Hq, h = bh % a.Hq, hk = h / a.group;
   const float *qp = (const float *)a.q + b * a.qs0 + h * a.qs1;
   const float *kp = (const float *)a.k + b * a.ks0 + hk * a.ks1;
   const float *vp = (const float *)a.v + b * a.vs0 + hk * a.vs1;
-  const int row = qb * F32_BM + rl;
+  const int row0 = qb * ROWS;
 
-  // rows past the end read the last row (never stored), so no load is
-  // guarded and all of them issue before the first is waited for
-  const int rowc = min(row, a.Sq - 1);
-  float q[D], acc[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    q[d] = qp[rowc * a.qs2 + d];
-    acc[d] = 0.0f;
-  }
-  float m = kNegFltMax, lsum = 0.0f;
-  int nkb = (a.Sk + BN - 1) / BN;
+  int nkb = (a.Sk + F32_KB - 1) / F32_KB;
   if (CAUSAL) {
-    int last = qb * F32_BM + F32_BM - 1 + a.off;
-    int lim = last < 0 ? 0 : last / BN + 1;
-    nkb = nkb < lim ? nkb : lim;
+    const int last = min(row0 + ROWS, a.Sq) - 1 + a.off;
+    nkb = min(nkb, last < 0 ? 0 : last / F32_KB + 1);
   }
-  constexpr int KPL = BN / F32_KS;  // keys per lane and block
-  for (int jb = 0; jb < nkb; ++jb) {
-    const int key0 = jb * BN;
-    __syncthreads();
-    // a fixed trip count, unrolled, so every element's load issues before
-    // the first one is waited for
-    static_assert(BN * D % F32_NT == 0, "whole staging rounds");
-    float kv[BN * D / F32_NT], vv[BN * D / F32_NT];
+
+  // rows and keys past the end read the last one (rows are not stored, keys
+  // are masked), so no load is guarded
+  f32x4 kf[NM];
+  auto load_k = [&](int kb) {
+    const float *r = kp + min(kb * F32_KB + i, a.Sk - 1) * a.ks2 + 4 * g;
 #pragma unroll
-    for (int i = 0; i < BN * D / F32_NT; ++i) {
-      const int e = t + i * F32_NT;
-      // keys past the end read the last key: their scores are masked to
-      // -inf, so their p is 0
-      const int r = e / D, c = e % D, key = min(key0 + r, a.Sk - 1);
-      kv[i] = kp[key * a.ks2 + c];
-      vv[i] = vp[key * a.vs2 + c];
+    for (int m = 0; m < NM; ++m) kf[m] = load_f32<4, VEC>(r + 16 * m);
+  };
+  load_k(w);
+  f32x4 qf[NQ][NM];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const float *r = qp + min(row0 + 16 * n + i, a.Sq - 1) * a.qs2 + 4 * g;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) qf[n][m] = load_f32<4, VEC>(r + 16 * m);
+  }
+
+  // O^T block c of query block n: element r is head_dim row 4 g + r of the
+  // block, which is head_dim VW (4 g + r) + c % VW + 64 (c / VW)
+  f32x4 o[NQ][NM];
+  float m[NQ], l[NQ];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    m[n] = kNegFltMax;
+    l[n] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NM; ++c) o[n][c] = f32x4{0, 0, 0, 0};
+  }
+  const float sc = a.scale2;
+
+  for (int kb = w; kb < nkb; kb += NW) {
+    const int key0 = kb * F32_KB;
+    VV vf[4][VL];  // V of keys 4 g + r
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float *vr = vp + min(key0 + 4 * g + r, a.Sk - 1) * a.vs2 + VW * i;
+#pragma unroll
+      for (int c = 0; c < VL; ++c) vf[r][c] = load_f32<VW, VEC>(vr + 64 * c);
+    }
+    // two chains of D / 2 terms per score: half the rounding of one chain of D,
+    // and no product waits for the one just before it
+    f32x4 s[NQ], s2[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) s[n] = s2[n] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < NM; c += 2)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          s[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qf[n][c][e], s[n], 0, 0, 0);
+          s2[n] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c + 1][e], qf[n][c + 1][e], s2[n], 0, 0, 0);
+        }
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[n][r] += s2[n][r];
+    // unconditionally (past the last block it re-reads the last key): a
+    // branch would make the compiler wait for these loads before P.V
+    load_k(kb + NW);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      if (key0 + F32_KB > a.Sk || (CAUSAL && key0 + F32_KB - 1 > row0 + 16 * n + a.off)) {
+        int lim = a.Sk - 1 - key0 - 4 * g;  // the lane's last visible r
+        if (CAUSAL) lim = min(lim, row0 + 16 * n + i + a.off - key0 - 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (r > lim) s[n][r] = -INFINITY;
+      }
+      // the running max moves only when a block's max passes it by more than
+      // 8 (log2 units): in between p <= 2^8, which fp32 holds as well. Past
+      // the first block it is formed only when a lane's sum says it may.
+      float rs = 0.0f;
+      f32x4 p;
+      auto expo = [&]() {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = fast_exp2(fmaf(s[n][r], sc, -m[n]));
+        rs = (p[0] + p[1]) + (p[2] + p[3]);
+      };
+      bool full = kb == w;
+      if (!full) {
+        expo();
+        full = __any(!(rs <= 256.0f));
+      }
+      if (full) {
+        const float mx = max_xor32(
+            max_xor16(fmaxf(fmaxf(s[n][0], s[n][1]), fmaxf(s[n][2], s[n][3]))));
+        const float m_blk = mx * sc;
+        if (__any(m_blk > m[n] + 8.0f)) {
+          const float m_new = fmaxf(m[n], m_blk);
+          const float alpha = fast_exp2(m[n] - m_new);
+          l[n] *= alpha;
+#pragma unroll
+          for (int c = 0; c < NM; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[n][c][r] *= alpha;
+          m[n] = m_new;
+        }
+        expo();
+      }
+      l[n] += rs;
+      s[n] = p;
     }
 #pragma unroll
-    for (int i = 0; i < BN * D / F32_NT; ++i) {
-      const int e = t + i * F32_NT;
-      Ks[e / D][e % D] = kv[i];
-      Vs[e / D][e % D] = vv[i];
-    }
-    __syncthreads();
-    float s[KPL];
-    float mx = -INFINITY;
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int jj = 0; jj < KPL; ++jj) {
-      const int j = F32_KS * jj + kl;
-      float dot = 0.0f;
+      for (int c = 0; c < NM; ++c)
 #pragma unroll
-      for (int d = 0; d < D; ++d) dot = fmaf(q[d], Ks[j][d], dot);
-      const int key = key0 + j;
-      float sv = dot * a.scale2;
-      if (key >= a.Sk || (CAUSAL && key > row + a.off)) sv = -INFINITY;
-      s[jj] = sv;
-      mx = fmaxf(mx, sv);
-    }
-    const float m_new = fmaxf(m, mx);
-    const float alpha = fast_exp2(m - m_new);
-    float rs = 0.0f;
+        for (int n = 0; n < NQ; ++n)
+          o[n][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][c / VW][c % VW], s[n][r], o[n][c],
+                                                         0, 0, 0);
+  }
+
+  // merge the waves' states
 #pragma unroll
-    for (int jj = 0; jj < KPL; ++jj) {
-      s[jj] = fast_exp2(s[jj] - m_new);
-      rs += s[jj];
-    }
-    lsum = lsum * alpha + rs;
-    m = m_new;
-#pragma unroll
-    for (int d = 0; d < D; ++d) acc[d] *= alpha;
-#pragma unroll
-    for (int jj = 0; jj < KPL; ++jj) {
-      const float pj = s[jj];
-      const int j = F32_KS * jj + kl;
-#pragma unroll
-      for (int d = 0; d < D; ++d) acc[d] = fmaf(pj, Vs[j][d], acc[d]);
+  for (int n = 0; n < NQ; ++n) {
+    l[n] += __shfl_xor(l[n], 16, 64);
+    l[n] += __shfl_xor(l[n], 32, 64);
+    if (g == 0) {
+      mm[w][16 * n + i] = m[n];
+      ml[w][16 * n + i] = l[n];
     }
   }
-  // merge the 16 lane states of the row (lanes rl * 16 .. rl * 16 + 15 of
-  // one wave): a lane that saw no visible key has m = -FLT_MAX and l = 0
-  const float M = row_max16(m);
-  const float wgt = fast_exp2(m - M);
-  const float ltot = row_sum16(lsum * wgt);
+  __syncthreads();
 #pragma unroll
-  for (int d = 0; d < D; ++d) acc[d] = row_sum16(acc[d] * wgt);
-  if (row < a.Sq && kl == 0) {
+  for (int n = 0; n < NQ; ++n) {
+    float M = kNegFltMax;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, mm[ww][16 * n + i]);
+    const float wgt = fast_exp2(m[n] - M);  // a wave with no visible key: l = 0, O = 0
+#pragma unroll
+    for (int c = 0; c < VL; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        VV v;
+#pragma unroll
+        for (int e = 0; e < VW; ++e) v[e] = o[n][c * VW + e][r] * wgt;
+        *(VV *)&mo[w][16 * n + i][64 * c + VW * (4 * g + r)] = v;
+      }
+  }
+  __syncthreads();
+  constexpr int CPR = D / 4;  // 16-byte chunks per row
+  for (int e = tid; e < ROWS * CPR; e += 64 * NW) {
+    const int rl = e / CPR, d = 4 * (e % CPR), row = row0 + rl;
+    if (row >= a.Sq) break;  // e, and with it the row, only grows
+    float M = kNegFltMax;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, mm[ww][rl]);
+    float ltot = 0.0f;
+    f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) {
+      ltot = fmaf(fast_exp2(mm[ww][rl] - M), ml[ww][rl], ltot);
+      const f32x4 v = *(const f32x4 *)&mo[ww][rl][d];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] += v[k];
+    }
     // the correctly rounded quotient acc / l (HTile:130-143): q = acc * (1/l)
     // with the correctly rounded reciprocal, then one residual step
     // q + fma(-q, l, acc) * (1/l) (Markstein's correction)
     const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
-    float *op = (float *)a.o + b * a.os0 + h * a.os1 + row * a.os2;
+    float *op = (float *)a.o + b * a.os0 + h * a.os1 + row * a.os2 + d;
+    f32x4 res;
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const float q0 = acc[d] * inv;
-      op[d] = __builtin_fmaf(__builtin_fmaf(-q0, ltot, acc[d]), inv, q0);
+    for (int k = 0; k < 4; ++k) {
+      const float q0 = acc[k] * inv;
+      res[k] = __builtin_fmaf(__builtin_fmaf(-q0, ltot, acc[k]), inv, q0);
     }
-    if (a.lse)
+    if constexpr (VEC) {
+      *(f32x4 *)op = res;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) op[k] = res[k];
+    }
+    if (a.lse && d == 0)
       a.lse[((int64_t)b * a.Hq + h) * a.Sq + row] =
           ltot > 0.0f ? (M + log2f(ltot)) * kLn2 : -INFINITY;
   }
@@ -396,12 +519,31 @@ void launch_mfma(const AttnArgs &args, bool causal, int grid, hipStream_t s) {
     hipLaunchKernelGGL((attn_fwd_mfma<E, D, false>), dim3(grid), dim3(NTHR), 0, s, args);
 }
 
-template <int D>
-void launch_f32(const AttnArgs &args, bool causal, int grid, hipStream_t s) {
-  if (causal)
-    hipLaunchKernelGGL((attn_fwd_f32<D, true>), dim3(grid), dim3(F32_NT), 0, s, args);
+template <int D, bool CAUSAL>
+void launch_f32_d(AttnArgs args, bool vec, hipStream_t s) {
+  auto go = [&](auto NQ, auto NW) {
+    constexpr int nq = decltype(NQ)::value, nw = decltype(NW)::value;
+    args.nqb = (args.Sq + 16 * nq - 1) / (16 * nq);
+    auto k = vec ? attn_fwd_f32<D, CAUSAL, nq, nw, true> : attn_fwd_f32<D, CAUSAL, nq, nw, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)(args.nqb * args.BH)), dim3(64 * nw), 0, s, args);
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  using I8 = std::integral_constant<int, 8>;
+  const int64_t groups = (int64_t)((args.Sq + 31) / 32) * args.BH;
+  if (groups >= (CAUSAL ? F32_FILL_CAUSAL : F32_FILL))
+    go(I2{}, I4{});
   else
-    hipLaunchKernelGGL((attn_fwd_f32<D, false>), dim3(grid), dim3(F32_NT), 0, s, args);
+    go(I1{}, I8{});
+}
+
+template <int D>
+void launch_f32(const AttnArgs &args, bool causal, bool vec, hipStream_t s) {
+  if (causal)
+    launch_f32_d<D, true>(args, vec, s);
+  else
+    launch_f32_d<D, false>(args, vec, s);
 }
 
 }  // namespace
@@ -448,9 +590,9 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
   }
   // a dispatch covers at most 2^32 - 1 work-items: one 256-thread work-group
   // per 128 query rows and (batch, head) (the most any 16-bit path launches),
-  // one 256-thread work-group per 16 rows for fp32
-  const int64_t rows = a.dtype == 0 ? F32_BM : BM, thr = a.dtype == 0 ? F32_NT : NTHR;
-  if ((a.seq_q + rows - 1) / rows * (a.batch * a.heads_q) * thr > (int64_t)0xffffffff) {
+  // one 256-thread work-group per 16 rows for fp32 (twice what it launches)
+  const int64_t rows = a.dtype == 0 ? 16 : BM;
+  if ((a.seq_q + rows - 1) / rows * (a.batch * a.heads_q) * NTHR > (int64_t)0xffffffff) {
     *why = "batch*heads*seq_q too large for one launch";
     return false;
   }
@@ -477,12 +619,14 @@ hipError_t launch_attn_fwd(const AttnLaunch &L, hipStream_t s) {
   a.scale2 = L.scale_log2;
   const bool causal = L.causal != 0;
   if (L.dtype == 0) {
-    a.nqb = (int32_t)((L.seq_q + F32_BM - 1) / F32_BM);
-    int grid = a.nqb * a.BH;
+    bool vec = true;
+    for (int i = 0; i < 3; ++i)
+      vec = vec && L.qs[i] % 4 == 0 && L.ks[i] % 4 == 0 && L.vs[i] % 4 == 0 && L.os[i] % 4 == 0;
+    for (const void *p : {L.q, L.k, L.v, (const void *)L.o}) vec = vec && ((uintptr_t)p & 15u) == 0;
     switch (L.head_dim) {
-      case 32: launch_f32<32>(a, causal, grid, s); break;
-      case 64: launch_f32<64>(a, causal, grid, s); break;
-      default: launch_f32<128>(a, causal, grid, s); break;
+      case 32: launch_f32<32>(a, causal, vec, s); break;
+      case 64: launch_f32<64>(a, causal, vec, s); break;
+      default: launch_f32<128>(a, causal, vec, s); break;
     }
   } else {
     a.nqb = (int32_t)((L.seq_q + BM - 1) / BM);
