@@ -22,4 +22,7 @@ struct AttnArgs {
 hipError_t launch_attn_d128(const AttnArgs &a, int32_t dtype, bool causal, int stages, bool kt,
                             hipStream_t s);
 
+// Launches the head_dim-64 16-bit kernel (attn_fwd_tile.hip).
+hipError_t launch_attn_d64(const AttnArgs &a, int32_t dtype, bool causal, hipStream_t s);
+
 }  // namespace neptune

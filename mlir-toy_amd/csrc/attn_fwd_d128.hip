@@ -20,12 +20,6 @@
 // stages the loads for blocks j+2 (K) and j+1 (V) are in flight during
 // iteration j.
 //
-// LDS tiles (K stored [.., seq, head_dim], and V) are 64 rows x 256 B of
-// 16-byte units, XOR-swizzled per row so that both the DMA writes (16 lanes
-// = one row) and the MFMA operand reads are bank-conflict free:
-//   K: unit u of row r at u ^ (r & 15)   (reads: 32 rows, one unit each)
-//   V: unit u of row r at u ^ 4(r & 3)   (transpose reads: 4 rows x 64 B)
-//
 // Knobs (template parameters, chosen per launch):
 //   STAGES (pipeline_stages, HTile:128): K and V tiles each have STAGES LDS
 //     slots and the loads run that many key blocks ahead of their use. 2 is
@@ -44,68 +38,14 @@
 // mask each runs one query block, and the grid dispatches the heaviest
 // blocks first, so the end of the launch is filled by the lightest ones.
 #include "attn_args.h"
-#include "device_common.h"
+#include "attn_tile.h"
 #include "kernels.h"
-#include "lds_dma.h"
 
 namespace neptune {
 namespace {
 
-constexpr int BM = 128;
-constexpr int BN = 64;
 constexpr int HD = 128;
-constexpr int NT = 256;
 constexpr int TILE = BN * HD * 2;  // bytes per K or V tile (16 KiB)
-constexpr float kSlack = 8.0f;     // lazy-rescale threshold (log2 units)
-constexpr float kSumCap = 256.0f;  // 2^kSlack: a lane's block sum at most this skips the max
-
-// Wave w copies rows [16w, 16w+16) of a 64 x 128 tile (four 1 KiB chunks of
-// four rows) straight into LDS. Full blocks take a wave-uniform base pointer
-// plus per-lane 32-bit offsets fixed for the whole kernel, so issuing a
-// chunk costs no vector ALU work; a block that runs past the end of the
-// sequence re-reads the last row instead (its scores are masked, so its P
-// is exactly 0).
-struct TileLoader {
-  const char *base;   // element (0, 0) of this (batch, head)
-  int64_t row_bytes;  // key stride in bytes
-  uint32_t off[4];    // per-lane byte offset of chunk c within a full block
-  int lane_row;       // 16 w + lane / 16: row of chunk 0 for this lane
-  int sw_base;        // lane & 15
-};
-
-template <bool IS_V>
-__device__ inline TileLoader make_loader(const uint16_t *src, int64_t stride, int w, int lane) {
-  TileLoader t;
-  t.base = (const char *)src;
-  t.row_bytes = stride * 2;
-  t.lane_row = 16 * w + (lane >> 4);
-  t.sw_base = lane & 15;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int r = t.lane_row + 4 * c;
-    const int unit = (lane & 15) ^ (IS_V ? ((r & 3) << 2) : (r & 15));
-    t.off[c] = (uint32_t)((int64_t)r * t.row_bytes + unit * 16);
-  }
-  return t;
-}
-
-template <bool IS_V>
-__device__ inline void tile_to_lds(const TileLoader &t, int key0, int Sk, const uint8_t *tile,
-                                   int w) {
-  if (key0 + BN <= Sk) {
-    const char *blk = t.base + (int64_t)key0 * t.row_bytes;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) dma16_sbase(blk, t.off[c], lds_offset(tile + (4 * w + c) * 1024));
-  } else {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int r = t.lane_row + 4 * c;
-      const int unit = t.sw_base ^ (IS_V ? ((r & 3) << 2) : (r & 15));
-      const int key = min(key0 + r, Sk - 1);
-      dma16(t.base + (int64_t)key * t.row_bytes + unit * 16, lds_offset(tile + (4 * w + c) * 1024));
-    }
-  }
-}
 
 // K stored [.., head_dim, seq]: a tile is 128 head_dim rows x 64 keys
 // (128 B). Wave w copies rows [32w, 32w+32) as four 1 KiB chunks of eight
@@ -148,18 +88,6 @@ __device__ inline void kt_tile_to_lds(const KtLoader &t, int key0, int Sk, const
             lds_offset(tile + (4 * w + c) * 1024));
     }
   }
-}
-
-__device__ inline void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
-
-// (lane, lane ^ 32) pair reductions through v_permlane32_swap
-__device__ inline float pair_max(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ inline float pair_sum(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // Work-group -> (batch*head, query blocks q0, q1; q1 == q0 for one block).
@@ -250,9 +178,9 @@ __global__ __launch_bounds__(NT, STAGES == 3 ? 1 : 2) void attn_fwd_d128(AttnArg
   const int n0 = nkb[0];
   const int nv = n0 + nkb[1];  // virtual key blocks: n0 for q0, then q1's
 
-  const TileLoader kl = make_loader<false>(kp, a.ks2, w, lane);
+  const TileLoader<HD> kl = make_loader<HD, false>(kp, a.ks2, w, lane);
   const KtLoader ktl = make_kt_loader(kp, a.ks2, w, lane);
-  const TileLoader vl = make_loader<true>(vp, a.vs2, w, lane);
+  const TileLoader<HD> vl = make_loader<HD, true>(vp, a.vs2, w, lane);
   // virtual block t -> key block of its query block
   auto vkey0 = [&](int t) { return (t < n0 ? t : t - n0) * BN; };
   auto load_k = [&](int t) {
