@@ -78,7 +78,8 @@ typedef struct neptune_backend_info {
  * of K and V tiles the kernel keeps in LDS per operand, i.e. how far its
  * loads run ahead (the htile.pipeline_stages loop attribute, HTile:128);
  * neither knob changes the result. Both apply to the head_dim-128 16-bit
- * kernel (0 = default elsewhere); k_dim_order = 1 needs seq_kv % 8 == 0. Query head h reads KV head h / (heads_q / heads_kv).
+ * kernel (0 = default elsewhere; launches too short to fill the GPU always
+ * keep two tiles); k_dim_order = 1 needs seq_kv % 8 == 0. Query head h reads KV head h / (heads_q / heads_kv).
  * Numerics follow tests/data/flash_attention_htile.mlir:23-143: scores are
  * scaled by scale_log2 (= log2(e)/sqrt(D) when 0, HTile:24) into the exp2
  * domain, the running max starts at -FLT_MAX, keys stream in blocks of 64,
@@ -168,6 +169,23 @@ NEPTUNE_API int32_t neptune_device_count(void);
 NEPTUNE_API neptune_status neptune_attn_fwd(const neptune_attn_desc *desc, const void *q,
                                 const void *k, const void *v, void *o,
                                 float *lse, void *stream);
+
+/* neptune_attn_fwd with a workspace, for launches too short to fill the GPU (few
+ * query rows over many keys: a prompt chunk over its cache, a few queries).
+ * Those cut their keys into splits that run side by side, keep each split's
+ * fp32 state (O~, m, l) in the workspace and merge them in the exp2 domain,
+ * as split-K decode does. neptune_attn_workspace_bytes gives the size (0: the
+ * launch is not split and workspace may be NULL); a smaller or missing
+ * workspace is NEPTUNE_ERR_WORKSPACE_TOO_SMALL. The workspace needs no
+ * clearing, must be 16-byte aligned and is in use until the call's work on
+ * `stream` is done. Arguments, results and errors are otherwise
+ * neptune_attn_fwd's; results differ from it by fp32 rounding of the sums. */
+NEPTUNE_API neptune_status neptune_attn_workspace_bytes(const neptune_attn_desc *desc,
+                                            size_t *bytes);
+
+NEPTUNE_API neptune_status neptune_attn_fwd_ws(const neptune_attn_desc *desc, const void *q,
+                                   const void *k, const void *v, void *o, float *lse,
+                                   void *workspace, size_t workspace_bytes, void *stream);
 
 /* ---- split-K decode ---------------------------------------------------- */
 

@@ -123,6 +123,89 @@ size_t decode_ws_bytes(const neptune_decode_desc *d, int64_t splits) {
   return align256(rows * d->head_dim * 4) + align256(rows * 2 * 4);
 }
 
+// the checks of an attention descriptor, and the launch it describes (no
+// tensors)
+neptune_status attn_resolve(const neptune_attn_desc *d, AttnLaunch *launch) {
+  if (!d) return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: desc is NULL");
+  if (d->batch <= 0 || d->heads_q <= 0 || d->heads_kv <= 0 || d->seq_q <= 0 ||
+      d->seq_kv <= 0 || d->head_dim <= 0)
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT,
+                "attn_fwd: sizes must be positive (batch=%lld heads_q=%lld heads_kv=%lld "
+                "seq_q=%lld seq_kv=%lld head_dim=%lld)",
+                (long long)d->batch, (long long)d->heads_q, (long long)d->heads_kv,
+                (long long)d->seq_q, (long long)d->seq_kv, (long long)d->head_dim);
+  if (d->heads_q % d->heads_kv)
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: heads_q (%lld) %% heads_kv (%lld) != 0",
+                (long long)d->heads_q, (long long)d->heads_kv);
+  if (d->dtype != NEPTUNE_DTYPE_F32 && d->dtype != NEPTUNE_DTYPE_F16 &&
+      d->dtype != NEPTUNE_DTYPE_BF16)
+    return fail(NEPTUNE_ERR_UNSUPPORTED, "attn_fwd: dtype %d (need F32, F16 or BF16)",
+                (int)d->dtype);
+  if (!(d->scale_log2 >= 0.0f) || !std::isfinite(d->scale_log2))
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: scale_log2 must be finite and >= 0");
+  if (d->pipeline_stages < 0 || d->pipeline_stages > 3)
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: pipeline_stages %d (need 0..3)",
+                (int)d->pipeline_stages);
+  if (d->k_dim_order != 0 && d->k_dim_order != 1)
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: k_dim_order %d (need 0 or 1)",
+                (int)d->k_dim_order);
+  AttnLaunch &L = *launch;
+  L.batch = d->batch; L.heads_q = d->heads_q; L.heads_kv = d->heads_kv;
+  L.seq_q = d->seq_q; L.seq_kv = d->seq_kv; L.head_dim = d->head_dim;
+  if (!resolve_strides(d->q_stride, d->heads_q, d->seq_q, d->head_dim, L.qs) ||
+      !(d->k_dim_order ? resolve_strides(d->k_stride, d->heads_kv, d->head_dim, d->seq_kv, L.ks)
+                       : resolve_strides(d->k_stride, d->heads_kv, d->seq_kv, d->head_dim, L.ks)) ||
+      !resolve_strides(d->v_stride, d->heads_kv, d->seq_kv, d->head_dim, L.vs) ||
+      !resolve_strides(d->o_stride, d->heads_q, d->seq_q, d->head_dim, L.os))
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT,
+                "attn_fwd: strides must be all zero (contiguous) or all positive");
+  L.dtype = d->dtype;
+  L.causal = d->causal ? 1 : 0;
+  L.stages = d->pipeline_stages ? d->pipeline_stages : 2;
+  L.k_dim_order = d->k_dim_order;
+  L.scale_log2 = d->scale_log2 != 0.0f
+                     ? d->scale_log2
+                     : (float)(1.4426950408889634 / std::sqrt((double)d->head_dim));
+  return NEPTUNE_OK;
+}
+
+// the attention entry points; ws: the caller has a workspace for the states of
+// split keys
+neptune_status attn_run(const neptune_attn_desc *d, const void *q, const void *k, const void *v,
+                        void *o, float *lse, bool ws, void *workspace, size_t workspace_bytes,
+                        void *stream) {
+  if (!d) return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: desc is NULL");
+  if (!q || !k || !v || !o)
+    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: q, k, v and o must be non-NULL");
+  AttnLaunch L;
+  neptune_status st = attn_resolve(d, &L);
+  if (st != NEPTUNE_OK) return st;
+  L.q = q; L.k = k; L.v = v; L.o = o; L.lse = lse;
+  if (d->dtype != NEPTUNE_DTYPE_F32) {
+    bool strides8 = true;
+    for (int i = 0; i < 3; ++i)
+      strides8 = strides8 && L.qs[i] % 8 == 0 && L.ks[i] % 8 == 0 && L.vs[i] % 8 == 0 &&
+                 L.os[i] % 8 == 0;
+    if (!strides8 || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
+      return fail(NEPTUNE_ERR_UNSUPPORTED,
+                  "attn_fwd: 16-bit tensors need 16-byte aligned base pointers and strides "
+                  "that are multiples of 8 elements");
+  }
+  const char *why = "";
+  if (!attn_supported(L, &why)) return fail(NEPTUNE_ERR_UNSUPPORTED, "attn_fwd: %s", why);
+  const AttnSplit split = attn_split(L, ws);
+  if (split.bytes) {
+    if (!workspace || workspace_bytes < split.bytes)
+      return fail(NEPTUNE_ERR_WORKSPACE_TOO_SMALL, "attn_fwd: workspace %zu bytes, need %zu",
+                  workspace ? workspace_bytes : (size_t)0, split.bytes);
+    if (!aligned16(workspace))
+      return fail(NEPTUNE_ERR_UNSUPPORTED, "attn_fwd: workspace must be 16-byte aligned");
+  }
+  st = device_ready();
+  if (st != NEPTUNE_OK) return st;
+  return hip_result(launch_attn_fwd(L, split, workspace, (hipStream_t)stream), "attn_fwd launch");
+}
+
 }  // namespace
 
 extern "C" {
@@ -148,64 +231,24 @@ int32_t neptune_device_count(void) {
 
 neptune_status neptune_attn_fwd(const neptune_attn_desc *d, const void *q, const void *k,
                                 const void *v, void *o, float *lse, void *stream) {
-  if (!d) return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: desc is NULL");
-  if (!q || !k || !v || !o)
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: q, k, v and o must be non-NULL");
-  if (d->batch <= 0 || d->heads_q <= 0 || d->heads_kv <= 0 || d->seq_q <= 0 ||
-      d->seq_kv <= 0 || d->head_dim <= 0)
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT,
-                "attn_fwd: sizes must be positive (batch=%lld heads_q=%lld heads_kv=%lld "
-                "seq_q=%lld seq_kv=%lld head_dim=%lld)",
-                (long long)d->batch, (long long)d->heads_q, (long long)d->heads_kv,
-                (long long)d->seq_q, (long long)d->seq_kv, (long long)d->head_dim);
-  if (d->heads_q % d->heads_kv)
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: heads_q (%lld) %% heads_kv (%lld) != 0",
-                (long long)d->heads_q, (long long)d->heads_kv);
-  if (d->dtype != NEPTUNE_DTYPE_F32 && d->dtype != NEPTUNE_DTYPE_F16 &&
-      d->dtype != NEPTUNE_DTYPE_BF16)
-    return fail(NEPTUNE_ERR_UNSUPPORTED, "attn_fwd: dtype %d (need F32, F16 or BF16)",
-                (int)d->dtype);
-  if (!(d->scale_log2 >= 0.0f) || !std::isfinite(d->scale_log2))
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: scale_log2 must be finite and >= 0");
-  if (d->pipeline_stages < 0 || d->pipeline_stages > 3)
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: pipeline_stages %d (need 0..3)",
-                (int)d->pipeline_stages);
-  if (d->k_dim_order != 0 && d->k_dim_order != 1)
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_fwd: k_dim_order %d (need 0 or 1)",
-                (int)d->k_dim_order);
+  return attn_run(d, q, k, v, o, lse, false, nullptr, 0, stream);
+}
+
+neptune_status neptune_attn_workspace_bytes(const neptune_attn_desc *d, size_t *bytes) {
+  if (!bytes) return fail(NEPTUNE_ERR_INVALID_ARGUMENT, "attn_workspace_bytes: bytes is NULL");
   AttnLaunch L;
-  L.q = q; L.k = k; L.v = v; L.o = o; L.lse = lse;
-  L.batch = d->batch; L.heads_q = d->heads_q; L.heads_kv = d->heads_kv;
-  L.seq_q = d->seq_q; L.seq_kv = d->seq_kv; L.head_dim = d->head_dim;
-  if (!resolve_strides(d->q_stride, d->heads_q, d->seq_q, d->head_dim, L.qs) ||
-      !(d->k_dim_order ? resolve_strides(d->k_stride, d->heads_kv, d->head_dim, d->seq_kv, L.ks)
-                       : resolve_strides(d->k_stride, d->heads_kv, d->seq_kv, d->head_dim, L.ks)) ||
-      !resolve_strides(d->v_stride, d->heads_kv, d->seq_kv, d->head_dim, L.vs) ||
-      !resolve_strides(d->o_stride, d->heads_q, d->seq_q, d->head_dim, L.os))
-    return fail(NEPTUNE_ERR_INVALID_ARGUMENT,
-                "attn_fwd: strides must be all zero (contiguous) or all positive");
-  L.dtype = d->dtype;
-  L.causal = d->causal ? 1 : 0;
-  L.stages = d->pipeline_stages ? d->pipeline_stages : 2;
-  L.k_dim_order = d->k_dim_order;
-  L.scale_log2 = d->scale_log2 != 0.0f
-                     ? d->scale_log2
-                     : (float)(1.4426950408889634 / std::sqrt((double)d->head_dim));
-  if (d->dtype != NEPTUNE_DTYPE_F32) {
-    bool strides8 = true;
-    for (int i = 0; i < 3; ++i)
-      strides8 = strides8 && L.qs[i] % 8 == 0 && L.ks[i] % 8 == 0 && L.vs[i] % 8 == 0 &&
-                 L.os[i] % 8 == 0;
-    if (!strides8 || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
-      return fail(NEPTUNE_ERR_UNSUPPORTED,
-                  "attn_fwd: 16-bit tensors need 16-byte aligned base pointers and strides "
-                  "that are multiples of 8 elements");
-  }
+  neptune_status st = attn_resolve(d, &L);
+  if (st != NEPTUNE_OK) return st;
   const char *why = "";
   if (!attn_supported(L, &why)) return fail(NEPTUNE_ERR_UNSUPPORTED, "attn_fwd: %s", why);
-  neptune_status st = device_ready();
-  if (st != NEPTUNE_OK) return st;
-  return hip_result(launch_attn_fwd(L, (hipStream_t)stream), "attn_fwd launch");
+  *bytes = attn_split(L, true).bytes;
+  return ok();
+}
+
+neptune_status neptune_attn_fwd_ws(const neptune_attn_desc *d, const void *q, const void *k,
+                                   const void *v, void *o, float *lse, void *workspace,
+                                   size_t workspace_bytes, void *stream) {
+  return attn_run(d, q, k, v, o, lse, true, workspace, workspace_bytes, stream);
 }
 
 neptune_status neptune_decode_workspace_bytes(const neptune_decode_desc *d, size_t *bytes) {

@@ -22,7 +22,21 @@ struct AttnArgs {
 hipError_t launch_attn_d128(const AttnArgs &a, int32_t dtype, bool causal, int stages, bool kt,
                             hipStream_t s);
 
-// Launches the head_dim-64 16-bit kernel (attn_fwd_tile.hip).
-hipError_t launch_attn_d64(const AttnArgs &a, int32_t dtype, bool causal, hipStream_t s);
+constexpr int kMaxAttnSplits = 32;  // a power of two (attn_combine)
+
+// Short launches: the keys cut into splits whose states attn_combine merges,
+// and (packed) the query heads of a KV head as one run of rows.
+struct SplitArgs {
+  int32_t nsplit;  // 0: the plain kernel; 1: no partials
+  int32_t kbs;     // 64-key blocks per split
+  int32_t packed;
+  float *po;       // [B * Hq * Sq, nsplit, head_dim]
+  float *pml;      // [B * Hq * Sq, nsplit, 2]: (m, l)
+};
+
+// Launches the kernels of attn_fwd_tile.hip: head_dim 64, or (x.nsplit > 0)
+// 64 or 128.
+hipError_t launch_attn_tile(const AttnArgs &a, const SplitArgs &x, int32_t dtype, int head_dim,
+                            bool causal, hipStream_t s);
 
 }  // namespace neptune

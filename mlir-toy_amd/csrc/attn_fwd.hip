@@ -9,6 +9,8 @@
 //
 // This file holds the fp32 kernel and the choice of kernel; the 16-bit ones
 // are attn_fwd_d128.hip (head_dim 128) and attn_fwd_tile.hip (head_dim 64).
+#include <algorithm>
+
 #include "device_common.h"
 #include "kernels.h"
 #include "attn_args.h"
@@ -365,7 +367,73 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
   return true;
 }
 
-hipError_t launch_attn_fwd(const AttnLaunch &L, hipStream_t s) {
+// The cut of a 16-bit launch that leaves the GPU short of work-groups (at 128
+// query rows each), by sizes alone:
+//
+// - Packing: the heads of a KV head share its K and V, so their rows may run
+//   on into one another's 128-row blocks. It is used when that takes fewer
+//   blocks, except under the causal mask over a long run of queries, where a
+//   block across two heads would see the keys of the later head's last rows.
+// - Splits: a work-group's time is its chain of 64-key blocks, so with at most
+//   one work-group per CU the chain is cut. The count is the one with the
+//   least estimated time, from what the kernels measured: a key block takes
+//   1.05 us alone on a CU and 1.65 us beside another work-group (head_dim 64:
+//   0.75 and 1.1), a launch 3 us, the combine 4.5 us, and the states
+//   move at 5 TB/s. A cut has to promise 5%. Measured (us, one piece /
+//   chosen cut / its count): 1 x 32/8 heads, 250 queries over 8000 keys 134 /
+//   44.5 / 8; 500 over 4000 71 / 44 / 4; 1 x 8 heads, 128 over 12000 197 / 22
+//   / 27; 8 x 32/4 heads, 1 over 4000 68 / 17 / 16; head_dim 64, 1 x 16/4,
+//   250 over 8000 99 / 23.6 / 8. Where it stays whole: 1 x 32 heads, 1000 over
+//   1000 causal 22.8 / 30.1 with two splits; 1 x 32/8, 256 over 512 13.9 / 17.1.
+// - Without the mask the head_dim-128 kernel runs two query blocks per
+//   work-group; up to 512 blocks they are better apart (1 x 4 heads, 512
+//   over 512: 25.0 / 13.4).
+AttnSplit attn_split(const AttnLaunch &L, bool partials) {
+  AttnSplit p;
+  if (L.dtype == 0 || L.k_dim_order != 0) return p;
+  const bool causal = L.causal != 0, d128 = L.head_dim == 128;
+  const int64_t group = L.heads_q / L.heads_kv, BHk = L.batch * L.heads_kv;
+  const int64_t rows = L.batch * L.heads_q * L.seq_q;
+  const int64_t plain = (L.seq_q + 127) / 128 * group * BHk;
+  const int64_t packed = (L.seq_q * group + 127) / 128 * BHk;
+  const int64_t nkb = (L.seq_kv + 63) / 64;
+  constexpr int64_t kSlots = 512;  // two work-groups on each of 256 CUs
+  p.packed = packed < plain && (!causal || L.seq_q < 128 || 4 * L.seq_q <= L.seq_kv);
+  const int64_t wgs = p.packed ? packed : plain;
+  // estimated nanoseconds with the keys cut into ns splits
+  auto cost = [&](int64_t ns) {
+    const int64_t step = wgs * ns <= kSlots / 2 ? (d128 ? 1050 : 750) : (d128 ? 1650 : 1100);
+    int64_t t = (nkb + ns - 1) / ns * step;
+    if (ns > 1) {
+      // states written and read: causal blocks leave the splits past them empty
+      const int64_t states = causal ? ns - (ns - 1) * std::min(L.seq_q, L.seq_kv) / (2 * L.seq_kv) : ns;
+      t += 3000 + 4500 + rows * states * (L.head_dim + 2) * 8 / 5000;
+    } else {
+      t += 3000;
+    }
+    return t;
+  };
+  int64_t best = 1;
+  if (partials && wgs <= kSlots / 2) {
+    const int64_t one = cost(1) * 95 / 100;
+    int64_t best_t = one;
+    for (int64_t ns = 2; ns <= kMaxAttnSplits && wgs * ns <= kSlots && ns <= nkb; ++ns)
+      if (cost(ns) < best_t) {
+        best_t = cost(ns);
+        best = ns;
+      }
+  }
+  if (best == 1 && !(p.packed && 2 * packed <= plain) &&
+      !(d128 && !causal && wgs <= kSlots))
+    return AttnSplit();
+  p.kbs = (int32_t)((nkb + best - 1) / best);
+  p.nsplit = (int32_t)((nkb + p.kbs - 1) / p.kbs);
+  if (p.nsplit > 1) p.bytes = (size_t)rows * p.nsplit * (L.head_dim + 2) * 4;
+  return p;
+}
+
+hipError_t launch_attn_fwd(const AttnLaunch &L, const AttnSplit &split, void *workspace,
+                           hipStream_t s) {
   AttnArgs a;
   a.q = L.q;
   a.k = L.k;
@@ -396,7 +464,15 @@ hipError_t launch_attn_fwd(const AttnLaunch &L, hipStream_t s) {
     }
   } else {
     a.nqb = (int32_t)((L.seq_q + 127) / 128);  // blocks of 128 query rows
-    if (L.head_dim == 64) return launch_attn_d64(a, L.dtype, causal, s);
+    if (split.nsplit > 0 || L.head_dim == 64) {
+      SplitArgs x;
+      x.nsplit = split.nsplit;
+      x.kbs = split.kbs;
+      x.packed = split.packed;
+      x.po = (float *)workspace;
+      x.pml = x.po + (size_t)(L.batch * L.heads_q * L.seq_q) * split.nsplit * L.head_dim;
+      return launch_attn_tile(a, x, L.dtype, (int)L.head_dim, causal, s);
+    }
     return launch_attn_d128(a, L.dtype, causal, L.stages, L.k_dim_order != 0, s);
   }
   return hipGetLastError();

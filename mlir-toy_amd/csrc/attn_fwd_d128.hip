@@ -37,6 +37,8 @@
 // while q0 drains, and a launch has half as many prologues. Under the causal
 // mask each runs one query block, and the grid dispatches the heaviest
 // blocks first, so the end of the launch is filled by the lightest ones.
+// Launches too short to fill the GPU go to attn_fwd_tile.hip, whatever their
+// stage count (attn_split in attn_fwd.hip).
 #include "attn_args.h"
 #include "attn_tile.h"
 #include "kernels.h"

@@ -1,4 +1,5 @@
-// attn_fwd_tile.hip — head_dim-64, 16-bit HTile attention forward for gfx950.
+// attn_fwd_tile.hip — 16-bit HTile attention forward for gfx950: head_dim 64,
+// and the cut form of short launches at head_dim 64 and 128.
 //
 // Semantics are those of attn_fwd.hip. The structure is that of the
 // head_dim-128 kernel (attn_fwd_d128.hip): 256 threads = 4 waves, 128 query
@@ -27,8 +28,13 @@
 namespace neptune {
 namespace {
 
-template <class E, int HD, bool CAUSAL>
-__global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a) {
+// SPLIT: a work-group takes one split of the keys (x.kbs blocks) and, packed,
+// rows that run through the heads of its KV head; with more than one split
+// it leaves its unnormalised O and (m, l) for attn_combine. 208 registers at
+// head_dim 128 (two work-groups per CU). What it measured stands at
+// attn_split, which chooses the cut.
+template <class E, int HD, bool CAUSAL, bool SPLIT>
+__global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) {
   typedef typename E::vec8 V8;
   constexpr int TILE = TileLoader<HD>::TILE_BYTES;
   constexpr int ROWB = HD * 2;   // bytes per LDS row
@@ -47,46 +53,80 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, g = lane >> 5;
 
-  // Work-group -> (kv head, query head of its group, query block): kv heads
-  // fastest, so that (with a multiple of 8 of them) id % 8, the XCD, fixes
-  // the kv head modulo 8 and all readers of a head's K and V share an L2;
-  // the heaviest causal query blocks first
+  // Work-group -> (kv head, split, query head of its group, query block): kv
+  // heads fastest, so that (with a multiple of 8 of them) id % 8, the XCD,
+  // fixes the kv head modulo 8 and all readers of a head's K and V share an
+  // L2; the heaviest causal query blocks first
   const int BHk = a.BH / a.group;
   const int id = blockIdx.x;
   const int bhk = __builtin_amdgcn_readfirstlane(id % BHk);
-  const int rest = id / BHk;
-  const int qb = __builtin_amdgcn_readfirstlane(a.nqb - 1 - rest / a.group);
+  int rest = id / BHk, split = 0;
+  if constexpr (SPLIT) {
+    split = __builtin_amdgcn_readfirstlane(rest % x.nsplit);
+    rest /= x.nsplit;
+  }
+  const bool packed = SPLIT && x.packed;
+  const int heads = packed ? 1 : a.group;  // work-groups per row block and kv head
+  const int qb = __builtin_amdgcn_readfirstlane(a.nqb - 1 - rest / heads);
   const int Hk = a.Hq / a.group;
   const int b = __builtin_amdgcn_readfirstlane(bhk / Hk);
   const int hk = bhk - b * Hk;
-  const int h = __builtin_amdgcn_readfirstlane(hk * a.group + rest % a.group);
-  const uint16_t *qp = (const uint16_t *)a.q + b * a.qs0 + h * a.qs1;
+  const int h0 = __builtin_amdgcn_readfirstlane(hk * a.group + rest % heads);
   const uint16_t *kp = (const uint16_t *)a.k + b * a.ks0 + hk * a.ks1;
   const uint16_t *vp = (const uint16_t *)a.v + b * a.vs0 + hk * a.vs1;
 
-  const int row0 = qb * BM + w * 32, row = row0 + lq;
-  // key blocks of the work-group and of this wave
-  int nv = (a.Sk + BN - 1) / BN, nkw = nv;
+  // this lane's row: query position pos of head h0 + hr (packed rows run
+  // through the heads of the group, each all its positions)
+  const int row = qb * BM + w * 32 + lq;
+  const int rows = packed ? a.group * a.Sq : a.Sq;
+  const int hr = packed ? row / a.Sq : 0, pos = row - hr * a.Sq;
+  // the first and last position among rows r0 .. r0 + n - 1
+  auto span = [&](int r0, int n, int *lo, int *hi) {
+    const int r1 = min(r0 + n, rows) - 1;
+    *lo = r0;
+    *hi = r1;
+    if (packed) {
+      const int p0 = r0 / a.Sq, p1 = r1 / a.Sq;
+      *lo = p0 == p1 ? r0 - p0 * a.Sq : 0;
+      *hi = p0 == p1 ? r1 - p1 * a.Sq : a.Sq - 1;
+    }
+  };
+  // key blocks kb0 .. kb0 + nv - 1 of the work-group, the first nkw of them
+  // this wave's
+  const int kb0 = SPLIT ? split * x.kbs : 0;
+  int nv = (a.Sk + BN - 1) / BN, nkw = nv, lo_w = 0;
   if (CAUSAL) {
-    const int last_wg = qb * BM + BM - 1 + a.off, last_w = row0 + 31 + a.off;
-    nv = min(nv, last_wg < 0 ? 0 : last_wg / BN + 1);
-    nkw = min(nv, last_w < 0 ? 0 : last_w / BN + 1);
+    int lo, hi;
+    span(qb * BM, BM, &lo, &hi);
+    nv = min(nv, hi + a.off < 0 ? 0 : (hi + a.off) / BN + 1);
+    span(qb * BM + w * 32, 32, &lo, &hi);
+    nkw = min(nv, hi + a.off < 0 ? 0 : (hi + a.off) / BN + 1);
+    lo_w = __builtin_amdgcn_readfirstlane(lo);
   }
+  if (qb * BM + w * 32 >= rows) nkw = 0;
+  if constexpr (SPLIT) {
+    nv = min(max(nv - kb0, 0), x.kbs);
+    nkw = min(max(nkw - kb0, 0), x.kbs);
+  }
+  nv = __builtin_amdgcn_readfirstlane(nv);
+  nkw = __builtin_amdgcn_readfirstlane(nkw);
 
   const TileLoader<HD> kl = make_loader<HD, false>(kp, a.ks2, w, lane);
   const TileLoader<HD> vl = make_loader<HD, true>(vp, a.vs2, w, lane);
-  auto load_k = [&](int t) { tile_to_lds<false>(kl, t * BN, a.Sk, kslot(t), w); };
-  auto load_v = [&](int t) { tile_to_lds<true>(vl, t * BN, a.Sk, vslot(t), w); };
+  auto load_k = [&](int t) { tile_to_lds<false>(kl, (kb0 + t) * BN, a.Sk, kslot(t), w); };
+  auto load_v = [&](int t) { tile_to_lds<true>(vl, (kb0 + t) * BN, a.Sk, vslot(t), w); };
   if (nv > 0) load_k(0);
   if (nv > 1) load_k(1);
   if (nv > 0) load_v(0);
 
   // Q^T operand: k-step st covers head_dim 16 st + 8 g .. +7 of the row
   u32x4 qf[NST];
+  {
+    const uint16_t *qp = (const uint16_t *)a.q + b * a.qs0 + (h0 + hr) * a.qs1 + pos * a.qs2 + 8 * g;
 #pragma unroll
-  for (int st = 0; st < NST; ++st)
-    qf[st] = row < a.Sq ? *(const u32x4 *)(qp + row * a.qs2 + 16 * st + 8 * g)
-                        : u32x4{0, 0, 0, 0};
+    for (int st = 0; st < NST; ++st)
+      qf[st] = row < rows ? *(const u32x4 *)(qp + 16 * st) : u32x4{0, 0, 0, 0};
+  }
 
   // per-lane LDS byte offsets of the operand reads
   int ka[NST];  // K: row lq (+32 kb), logical unit 2 st + g
@@ -153,12 +193,12 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a) {
       // the first two V^T operands of this block's P.V, read before the softmax
       const uint8_t *vt = vslot(jb);
       const u32x4 vp0 = v_operand(vt, 0), vp1 = v_operand(vt, 1);
-      const int key0 = jb * BN;
-      if ((key0 + BN > a.Sk) || (CAUSAL && key0 + BN - 1 > row0 + a.off)) {
+      const int key0 = (kb0 + jb) * BN;
+      if ((key0 + BN > a.Sk) || (CAUSAL && key0 + BN - 1 > lo_w + a.off)) {
         // element (kb, r) holds key key0 + 4 g + c with c = 32 kb + 8 (r >> 2)
         // + (r & 3): it is masked when c passes the lane's last visible key
         int lim = a.Sk - 1 - key0 - 4 * g;
-        if (CAUSAL) lim = min(lim, row + a.off - key0 - 4 * g);
+        if (CAUSAL) lim = min(lim, pos + a.off - key0 - 4 * g);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -240,46 +280,143 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a) {
     __syncthreads();
   }
 
-  // O = acc / l rounded to the input type (HTile:130-143), the correctly
-  // rounded fp32 quotient by Markstein's correction, and the LSE
   const float ltot = pair_sum(lsum);
-  if (row < a.Sq) {
+  if (row < rows) {
+    const int64_t grow = ((int64_t)b * a.Hq + h0 + hr) * a.Sq + pos;  // row of [B, Hq, Sq]
+    if constexpr (SPLIT) {
+      if (x.nsplit > 1) {  // this split's state, for attn_combine
+        const int64_t part = grow * x.nsplit + split;
+        if (nv > 0) {
+          float *op = x.po + part * HD + 4 * g;
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int rq = 0; rq < 4; ++rq)
+              *(f32x4 *)(op + 32 * nb + 8 * rq) =
+                  f32x4{o[nb][4 * rq], o[nb][4 * rq + 1], o[nb][4 * rq + 2], o[nb][4 * rq + 3]};
+        }
+        if (g == 0) *(f32x2 *)(x.pml + part * 2) = f32x2{m, ltot};
+        return;
+      }
+    }
+    // O = acc / l rounded to the input type (HTile:130-143), the correctly
+    // rounded fp32 quotient by Markstein's correction, and the LSE
     const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
-    auto quot = [&](float x) {
-      const float q0 = x * inv;
-      return __builtin_fmaf(__builtin_fmaf(-q0, ltot, x), inv, q0);
+    auto quot = [&](float v) {
+      const float q0 = v * inv;
+      return __builtin_fmaf(__builtin_fmaf(-q0, ltot, v), inv, q0);
     };
-    uint16_t *op = (uint16_t *)a.o + b * a.os0 + h * a.os1 + row * a.os2;
+    uint16_t *op = (uint16_t *)a.o + b * a.os0 + (h0 + hr) * a.os1 + pos * a.os2 + 4 * g;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
         const u32x2 pk = {E::pack2(quot(o[nb][4 * rq]), quot(o[nb][4 * rq + 1])),
                           E::pack2(quot(o[nb][4 * rq + 2]), quot(o[nb][4 * rq + 3]))};
-        *(u32x2 *)(op + 32 * nb + 8 * rq + 4 * g) = pk;
+        *(u32x2 *)(op + 32 * nb + 8 * rq) = pk;
       }
     if (g == 0 && a.lse)
-      a.lse[((int64_t)b * a.Hq + h) * a.Sq + row] =
-          ltot > 0.0f ? (m + log2f(ltot)) * kLn2 : -INFINITY;
+      a.lse[grow] = ltot > 0.0f ? (m + log2f(ltot)) * kLn2 : -INFINITY;
+  }
+}
+
+// Combine of the splits' states: HD / 4 lanes per row, four head_dim elements
+// each. M = max m_s, l = sum 2^(m_s - M) l_s, O = sum 2^(m_s - M) O_s / l; a
+// split with l_s = 0 (no visible key) has left no O_s. NS (a power of two) is
+// at least the number of splits: every O_s is loaded before the first weight
+// is known, so the row waits on memory once.
+template <class E, int HD, int NS>
+__global__ __launch_bounds__(NT) void attn_combine(AttnArgs a, SplitArgs x, int64_t nrows) {
+  constexpr int LPR = HD / 4;
+  const int64_t grow0 = (int64_t)blockIdx.x * (NT / LPR) + threadIdx.x / LPR;
+  const int64_t grow = grow0 < nrows ? grow0 : nrows - 1;  // every lane takes part in the shuffles
+  const int dl = threadIdx.x % LPR, d = 4 * dl;
+  const f32x2 *ml = (const f32x2 *)x.pml + grow * x.nsplit;
+  const float *po = x.po + grow * x.nsplit * HD + d;
+  f32x4 os[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) os[s] = *(const f32x4 *)(po + (int64_t)min(s, x.nsplit - 1) * HD);
+  // lane dl holds the state of splits dl, dl + LPR, ..
+  constexpr int SPL = (NS + LPR - 1) / LPR;
+  f32x2 st[SPL];
+  float M = kNegFltMax;
+#pragma unroll
+  for (int i = 0; i < SPL; ++i) {
+    const int s = dl + i * LPR;
+    st[i] = s < x.nsplit ? ml[s] : f32x2{kNegFltMax, 0.0f};
+    M = fmaxf(M, st[i][0]);
+  }
+#pragma unroll
+  for (int off = LPR / 2; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, LPR));
+  float l = 0.0f;
+#pragma unroll
+  for (int i = 0; i < SPL; ++i) {
+    st[i][0] = st[i][1] == 0.0f ? 0.0f : fast_exp2(st[i][0] - M);  // the split's weight
+    l = fmaf(st[i][0], st[i][1], l);
+  }
+#pragma unroll
+  for (int off = LPR / 2; off >= 1; off >>= 1) l += __shfl_xor(l, off, LPR);
+  f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const float wgt = __shfl(st[s / LPR][0], s % LPR, LPR);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = wgt == 0.0f ? acc[k] : fmaf(wgt, os[s][k], acc[k]);
+  }
+  if (grow0 >= nrows) return;
+  const int64_t bh = grow / a.Sq;
+  const int pos = (int)(grow - bh * a.Sq), b = (int)(bh / a.Hq), h = (int)(bh - (int64_t)b * a.Hq);
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  auto quot = [&](float v) {
+    const float q0 = v * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q0, l, v), inv, q0);
+  };
+  uint16_t *op = (uint16_t *)a.o + b * a.os0 + h * a.os1 + pos * a.os2 + d;
+  *(u32x2 *)op = u32x2{E::pack2(quot(acc[0]), quot(acc[1])), E::pack2(quot(acc[2]), quot(acc[3]))};
+  if (d == 0 && a.lse) a.lse[grow] = l > 0.0f ? (M + log2f(l)) * kLn2 : -INFINITY;
+}
+
+template <class E, int HD, bool CAUSAL>
+void launch_split(AttnArgs a, const SplitArgs &x, hipStream_t s) {
+  const int BHk = a.BH / a.group;
+  const int rows = x.packed ? a.group * a.Sq : a.Sq;
+  a.nqb = (rows + BM - 1) / BM;
+  const unsigned grid = (unsigned)a.nqb * (x.packed ? BHk : a.BH) * x.nsplit;
+  hipLaunchKernelGGL((attn_fwd_tile<E, HD, CAUSAL, true>), dim3(grid), dim3(NT), 0, s, a, x);
+  if (x.nsplit > 1) {
+    const int64_t nrows = (int64_t)a.BH * a.Sq, per = NT / (HD / 4);
+    auto k = x.nsplit <= 4    ? attn_combine<E, HD, 4>
+             : x.nsplit <= 8  ? attn_combine<E, HD, 8>
+             : x.nsplit <= 16 ? attn_combine<E, HD, 16>
+                              : attn_combine<E, HD, kMaxAttnSplits>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((nrows + per - 1) / per)), dim3(NT), 0, s, a, x, nrows);
   }
 }
 
 template <class E>
-void launch_e(const AttnArgs &a, bool causal, hipStream_t s) {
+void launch_e(const AttnArgs &a, const SplitArgs &x, int head_dim, bool causal, hipStream_t s) {
+  if (x.nsplit > 0) {
+    if (head_dim == 64)
+      causal ? launch_split<E, 64, true>(a, x, s) : launch_split<E, 64, false>(a, x, s);
+    else
+      causal ? launch_split<E, 128, true>(a, x, s) : launch_split<E, 128, false>(a, x, s);
+    return;
+  }
   const dim3 grid((unsigned)(a.nqb * a.BH));
   if (causal)
-    hipLaunchKernelGGL((attn_fwd_tile<E, 64, true>), grid, dim3(NT), 0, s, a);
+    hipLaunchKernelGGL((attn_fwd_tile<E, 64, true, false>), grid, dim3(NT), 0, s, a, x);
   else
-    hipLaunchKernelGGL((attn_fwd_tile<E, 64, false>), grid, dim3(NT), 0, s, a);
+    hipLaunchKernelGGL((attn_fwd_tile<E, 64, false, false>), grid, dim3(NT), 0, s, a, x);
 }
 
 }  // namespace
 
-hipError_t launch_attn_d64(const AttnArgs &a, int32_t dtype, bool causal, hipStream_t s) {
+hipError_t launch_attn_tile(const AttnArgs &a, const SplitArgs &x, int32_t dtype, int head_dim,
+                            bool causal, hipStream_t s) {
   if (dtype == 2)
-    launch_e<Bf16Tag>(a, causal, s);
+    launch_e<Bf16Tag>(a, x, head_dim, causal, s);
   else
-    launch_e<F16Tag>(a, causal, s);
+    launch_e<F16Tag>(a, x, head_dim, causal, s);
   return hipGetLastError();
 }
 

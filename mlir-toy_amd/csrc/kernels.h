@@ -20,6 +20,15 @@ struct AttnLaunch {
   int32_t k_dim_order;  // 1: K is [batch, head, head_dim, seq]; ks[2] = head_dim-row stride
 };
 
+// How a short 16-bit attention launch is cut further (attn_split); nsplit 0:
+// it is not.
+struct AttnSplit {
+  int32_t nsplit = 0;  // key splits (1: none, the rows are packed only)
+  int32_t kbs = 0;     // 64-key blocks per split
+  int32_t packed = 0;  // the query heads of a KV head form one run of rows
+  size_t bytes = 0;    // workspace the splits' states take
+};
+
 struct DecodeLaunch {
   const void *q, *k, *v;
   const float *k_scale, *v_scale;  // fp8 only
@@ -64,10 +73,15 @@ hipError_t decode_scratch(hipStream_t s, void **ptr);
 
 // Each returns hipSuccess or the launch error. Shapes the kernels do not
 // cover are rejected by the ABI layer before these are called.
-hipError_t launch_attn_fwd(const AttnLaunch &a, hipStream_t s);
+hipError_t launch_attn_fwd(const AttnLaunch &a, const AttnSplit &split, void *workspace,
+                           hipStream_t s);
 hipError_t launch_decode(const DecodeLaunch &a, hipStream_t s);
 hipError_t launch_kv_quantize(const QuantLaunch &a, hipStream_t s);
 hipError_t launch_selective_scan(const ScanLaunch &a, hipStream_t s);
+
+// The cut for a launch the library covers; `partials`: a workspace for the
+// splits' states is to be had.
+AttnSplit attn_split(const AttnLaunch &a, bool partials);
 
 // Coverage predicates used by the ABI layer for NEPTUNE_ERR_UNSUPPORTED.
 bool attn_supported(const AttnLaunch &a, const char **why);

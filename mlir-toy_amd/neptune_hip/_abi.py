@@ -40,6 +40,8 @@ EXPORTED_SYMBOLS = (
     "neptune_last_error",
     "neptune_device_count",
     "neptune_attn_fwd",
+    "neptune_attn_workspace_bytes",
+    "neptune_attn_fwd_ws",
     "neptune_decode_workspace_bytes",
     "neptune_decode_splitk",
     "neptune_decode_splitk_noalloc",
@@ -186,6 +188,15 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.neptune_device_count.restype = i32
     lib.neptune_attn_fwd.argtypes = [ctypes.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp]
     lib.neptune_attn_fwd.restype = i32
+    lib.neptune_attn_workspace_bytes.argtypes = [
+        ctypes.POINTER(AttnDesc),
+        ctypes.POINTER(ctypes.c_size_t),
+    ]
+    lib.neptune_attn_workspace_bytes.restype = i32
+    lib.neptune_attn_fwd_ws.argtypes = [
+        ctypes.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp, ctypes.c_size_t, vp,
+    ]
+    lib.neptune_attn_fwd_ws.restype = i32
     lib.neptune_decode_workspace_bytes.argtypes = [
         ctypes.POINTER(DecodeDesc),
         ctypes.POINTER(ctypes.c_size_t),

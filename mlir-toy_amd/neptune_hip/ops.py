@@ -8,6 +8,7 @@ fallback path: if the library is missing, ``load_library`` raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -58,6 +59,21 @@ def scale_to_log2(scale: float | None, head_dim: int) -> float:
     if scale is None:
         return 0.0  # library default: log2(e)/sqrt(head_dim), HTile:24
     return float(scale) * LOG2E
+
+
+@functools.lru_cache(maxsize=1024)
+def _attn_workspace_bytes(B, Hq, Hk, Sq, Sk, D, dtype, causal, stages, k_dim_order) -> int:
+    """neptune_attn_workspace_bytes, a function of these sizes alone; 0 for
+    what the library refuses, which the launch itself then reports."""
+    desc = _abi.AttnDesc()
+    desc.batch, desc.heads_q, desc.heads_kv = B, Hq, Hk
+    desc.seq_q, desc.seq_kv, desc.head_dim = Sq, Sk, D
+    desc.dtype, desc.causal = dtype, causal
+    desc.pipeline_stages, desc.k_dim_order = stages, k_dim_order
+    n = ctypes.c_size_t()
+    lib = load_library()
+    st = lib.neptune_attn_workspace_bytes(ctypes.byref(desc), ctypes.byref(n))
+    return n.value if st == _abi.OK else 0
 
 
 def attention(
@@ -122,15 +138,22 @@ def attention(
     desc.pipeline_stages = int(pipeline_stages)
     desc.k_dim_order = int(k_dim_order)
     lib = load_library()
+    # states of split keys (short launches only): held by the caching allocator
+    # until the current stream is past this call
+    n = _attn_workspace_bytes(B, Hq, Hk, Sq, Sk, D, desc.dtype, desc.causal, desc.pipeline_stages,
+                              desc.k_dim_order)
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
     with torch.cuda.device(q.device):
         check(
-            lib.neptune_attn_fwd(
+            lib.neptune_attn_fwd_ws(
                 ctypes.byref(desc),
                 q.data_ptr(),
                 k.data_ptr(),
                 v.data_ptr(),
                 out.data_ptr(),
                 lse.data_ptr() if lse is not None else None,
+                ws.data_ptr() if ws is not None else None,
+                n,
                 _stream(q),
             ),
             lib,
