@@ -67,8 +67,8 @@
 // their own steps, whose outputs are not stored, and the last chunk's end
 // state is never read, so whatever they compute goes nowhere.
 //
-// Sequence-parallel path. When batch * dim / 16 work-groups cannot fill the
-// GPU (few channels, long sequences), the sequence is cut into nch chunks of
+// Sequence-parallel path. When batch * dim / 16 work-groups leave CUs empty
+// (few channels, long sequences), the sequence is cut into nch chunks of
 // nearly equal length (whole 32-step units, at least two per chunk) and the
 // scan runs in three launches, using y itself as scratch (no workspace):
 //   state   every chunk but the last scans from x = 0 without outputs and
@@ -113,15 +113,19 @@ struct ScanArgs {
 // the output kernel as the single pass, and as the chunked path's output pass
 enum ScanMode { kScanFull = 0, kScanOutput = 1 };
 
-// chunk k of channel d of batch row b: its y segment as fp32 scratch
-// (x[16], then S)
+// chunk k of channel d of batch row b: its y segment (64 steps or more) as
+// fp32 scratch (x[16], then S), from the segment's first multiple of 4 bytes
+// (as far into every segment of a row: chunks start 64 bytes apart)
 __device__ inline int chunk_start(const ScanArgs &a, int k) {
   return TT * (k * a.Tu + min(k, a.rem));
 }
-__device__ inline float *chunk_scratch(const ScanArgs &a, int b, int d, int k) {
-  return reinterpret_cast<float *>(a.y + ((int64_t)b * a.Dm + d) * a.L + chunk_start(a, k));
+__device__ inline float *row_scratch(const ScanArgs &a, int b, int d) {
+  uint16_t *p = a.y + ((int64_t)b * a.Dm + d) * a.L;
+  return reinterpret_cast<float *>(p + ((uintptr_t)p >> 1 & 1));
 }
-
+__device__ inline float *chunk_scratch(const ScanArgs &a, float *row, int k) {
+  return row + chunk_start(a, k) / 2;
+}
 
 
 __device__ inline float silu_fast(float z) {
@@ -134,7 +138,7 @@ constexpr float kSoftplusLinear2 = 20.0f * kLog2e;
 // The state pass of the chunked path: the recurrence alone, from x = 0, over
 // every chunk but the last; leaves the chunk's end state and delta sum at
 // the start of its own y segment.
-template <bool SOFTPLUS>
+template <bool SOFTPLUS, bool PAIRS>
 __global__ __launch_bounds__(NT) void selective_scan_state(ScanArgs a) {
   // (delta log2 e, delta u) for two steps per float4, and B of one state for
   // two steps, double-buffered by chunk parity (one barrier per chunk); one
@@ -176,14 +180,19 @@ __global__ __launch_bounds__(NT) void selective_scan_state(ScanArgs a) {
   const float bias2 = (sok && a.bias) ? a.bias[sd] * kLog2e : 0.0f;
 
   // every chunk of this pass lies inside the sequence, and so does the step
-  // pair after it (the last chunk follows), so the loads need no guard; the
-  // path needs even L and 4-byte aligned rows, so a step pair is one dword
+  // pair after it (the last chunk follows), so the loads need no guard. With
+  // PAIRS (even L, 4-byte aligned rows) a step pair is one dword, otherwise
+  // two 16-bit loads
   uint32_t pu, pdr, pB;
+  auto pair = [](const uint16_t *p) {
+    if constexpr (PAIRS) return *(const uint32_t *)p;
+    return (uint32_t)p[0] | (uint32_t)p[1] << 16;
+  };
   auto fetch = [&](int t0) {
     const int t = t0 + 2 * sp;
-    pu = *(const uint32_t *)(a.u + srow + t);
-    pdr = *(const uint32_t *)(a.dr + srow + t);
-    pB = *(const uint32_t *)(a.Bm + bcrow + t);
+    pu = pair(a.u + srow + t);
+    pdr = pair(a.dr + srow + t);
+    pB = pair(a.Bm + bcrow + t);
   };
 
   fetch(tb);
@@ -219,10 +228,10 @@ __global__ __launch_bounds__(NT) void selective_scan_state(ScanArgs a) {
       x = fmaf(fast_exp2(pd.z * Ac), x, pd.w * q.y);
     }
   }
-  if (cok) chunk_scratch(a, b, d0 + c, kc)[n] = x;
+  if (cok) chunk_scratch(a, row_scratch(a, b, d0 + c), kc)[n] = x;
 #pragma unroll
   for (int off = 1; off < TP; off <<= 1) dsum += __shfl_xor(dsum, off, 64);
-  if (sok && sp == 0) chunk_scratch(a, b, sd, kc)[ST] = dsum * kLn2;  // natural units
+  if (sok && sp == 0) chunk_scratch(a, row_scratch(a, b, sd), kc)[ST] = dsum * kLn2;  // natural units
 }
 
 // Cross-lane exchange through LDS inside one wave: the wave's LDS
@@ -317,7 +326,7 @@ __global__ __launch_bounds__(NT, 5) void selective_scan_out(ScanArgs a) {
   // this chunk's segment; every thread holds it (the load retired, below)
   // before the first barrier, and the work-group's first store follows that
   // barrier
-  float x = (MODE == kScanOutput && cok) ? chunk_scratch(a, b, ch, kc)[n] : 0.0f;
+  float x = (MODE == kScanOutput && cok) ? chunk_scratch(a, row_scratch(a, b, ch), kc)[n] : 0.0f;
   const float bias2 = (cok && a.bias) ? a.bias[ch] * kLog2e : 0.0f;
   const float D2 = (cok && a.D) ? a.D[ch] * kLog2e : 0.0f;  // times u ln2: D u
   // B / C identity: state bn, steps 2 sp and 2 sp + 1
@@ -495,6 +504,7 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
   if (gid >= lanes) return;
   const int n = gid & (ST - 1), bd = gid / ST;
   const int b = bd / a.Dm, d = bd - b * a.Dm;
+  float *const row_s = row_scratch(a, b, d);
   const float A2 = a.A[(int64_t)d * ST + n] * kLog2e;
   const int nsum = a.nch - 1;  // chunks with a summary: all but the last
   float xe[2][KB], S[2][KB];
@@ -503,7 +513,7 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
 #pragma unroll
     for (int i = 0; i < KB; ++i) {
       // past the last summary: re-read it (the value is not used)
-      const float *p = chunk_scratch(a, b, d, min(k0 + i, nsum - 1));
+      const float *p = chunk_scratch(a, row_s, min(k0 + i, nsum - 1));
       xe[set][i] = p[n];
       S[set][i] = p[ST];
     }
@@ -514,7 +524,7 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
 #pragma unroll
     for (int i = 0; i < KB; ++i)
       if (k0 + i < nsum) {
-        chunk_scratch(a, b, d, k0 + i)[n] = carry;
+        chunk_scratch(a, row_s, k0 + i)[n] = carry;
         carry = fmaf(fast_exp2(A2 * S[set][i]), carry, xe[set][i]);
       }
   };
@@ -527,7 +537,7 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
     load(S0{}, k0 + 2 * KB);
     walk(S1{}, k0 + KB);
   }
-  chunk_scratch(a, b, d, nsum)[n] = carry;  // the last chunk's starting state
+  chunk_scratch(a, row_s, nsum)[n] = carry;  // the last chunk's starting state
 }
 
 // The carry pass for long chains of chunks (more than 64 summaries): one
@@ -545,13 +555,14 @@ __global__ __launch_bounds__(256) void selective_scan_carry_wave(ScanArgs a, int
   const int lane = threadIdx.x & 63;
   const int n = row & (ST - 1), bd = row / ST;
   const int b = bd / a.Dm, d = bd - b * a.Dm;
+  float *const row_s = row_scratch(a, b, d);
   const float A2 = a.A[(int64_t)d * ST + n] * kLog2e;
   const int nsum = a.nch - 1;
   float carry = 0.0f;  // the state at the start of the pass (the same in every lane)
   for (int k0 = 0; k0 < nsum; k0 += 64) {
     const int k = k0 + lane;
     const bool live = k < nsum;
-    const float *p = chunk_scratch(a, b, d, live ? k : nsum - 1);
+    const float *p = chunk_scratch(a, row_s, live ? k : nsum - 1);
     float m = live ? fast_exp2(A2 * p[ST]) : 1.0f;  // this lane's map: x -> m x + c
     float c = live ? p[n] : 0.0f;
 #pragma unroll
@@ -566,40 +577,60 @@ __global__ __launch_bounds__(256) void selective_scan_carry_wave(ScanArgs a, int
     // this chunk starts where the lanes before it end
     const float mp = __shfl_up(m, 1, 64), cp = __shfl_up(c, 1, 64);
     const float start = lane == 0 ? carry : fmaf(mp, carry, cp);
-    if (live) chunk_scratch(a, b, d, k)[n] = start;
+    if (live) chunk_scratch(a, row_s, k)[n] = start;
     carry = fmaf(__shfl(m, 63, 64), carry, __shfl(c, 63, 64));
   }
-  if (lane == 0) chunk_scratch(a, b, d, nsum)[n] = carry;  // the last chunk's starting state
+  if (lane == 0) chunk_scratch(a, row_s, nsum)[n] = carry;  // the last chunk's starting state
 }
 
 }  // namespace
 
-// Chunking of the sequence-parallel path: used when the single pass would
-// launch fewer than kScanFillGroups work-groups (four per CU) and the
-// sequence holds at least two 64-step chunks; the chunk count brings the
-// launch to about kScanTargetGroups work-groups (five per CU, what the
-// single pass gets at config 4). The whole 32-step units of the sequence
-// are dealt out evenly: every chunk holds Tu or Tu + 1 units (Tu >= 2), the
-// last one also the partial unit at the end, so no chunk holds up its
-// launch by more than 32 steps. nch = 1: the single pass. The chunked path
-// needs the 4-byte pair access (even L).
-constexpr int64_t kScanFillGroups = 1024, kScanTargetGroups = 1280, kScanMinChunk = 64;
+// Chunking of the sequence-parallel path, by sizes alone: the chunk count
+// with the least estimated time, the single pass (nch = 1) among them. The
+// whole 32-step units of the sequence are dealt out evenly: every chunk holds
+// Tu or Tu + 1 units (Tu >= 2), the last one also the partial unit at the
+// end, so no chunk holds up its launch by more than 32 steps.
+//
+// The estimates are what the kernels measured: with k work-groups on the
+// busiest CU a unit of the output kernel takes 0.60 + 0.43 k us (1.03 alone,
+// 2.75 at the five that fit) and one of the state kernel 0.35 + 0.33 k; a
+// launch adds 2.5 us and the carry pass 4. A CU already holding two
+// work-groups of the single pass gains nothing from chunks, which do 1.6
+// times the work; and chunks past 1280 work-groups (five per CU) would run a
+// second round for a few. Measured (us, single / the count chosen here): B1
+// D2048 L2047 69.3 / 41.4, B3 D444 L817 29.1 / 19.6, B6 D660 L4637 153 / 130; where the single pass stays, against chunks: B2 D3511 L3465 150 / 179,
+// B1 D2260 L539 20.0 / 22.6, B2 D548 L227 10.4 / 14.2.
+constexpr int64_t kScanFillGroups = 1024, kScanMaxGroups = 1280, kScanMinUnits = 2;
 constexpr int64_t kScanMaxSeq = (int64_t)1 << 26;  // 16 rows x 2 bytes x 2^26 = 2^31
 
-void scan_chunking(int64_t batch, int64_t dim, int64_t L, bool vec, int32_t *Tu, int32_t *rem,
+void scan_chunking(int64_t batch, int64_t dim, int64_t L, int32_t *Tu, int32_t *rem,
                    int32_t *nch) {
   const int64_t groups = (dim + SCH - 1) / SCH * batch;
   *Tu = 0;
   *rem = 0;
   *nch = 1;
-  if (!vec || groups >= kScanFillGroups || L < 2 * kScanMinChunk) return;
   const int64_t units = L / TT;
-  int64_t want = (kScanTargetGroups + groups - 1) / groups;
-  want = std::min(want, units / (kScanMinChunk / TT));
-  if (want < 2) return;
-  *nch = (int32_t)want;
-  *Tu = (int32_t)(units / want);
-  *rem = (int32_t)(units % want);
+  if (groups >= kScanFillGroups || units < 2 * kScanMinUnits) return;
+  // estimated nanoseconds of n chunks: the longest chunk's steps of the
+  // state pass and of the output
+  auto cost = [&](int64_t n) {
+    const int64_t state = TT * (units / n + (units % n != 0));
+    const int64_t out = std::max(state, TT * (units / n) + L % TT);
+    int64_t t = 2500 + out * (600 + 430 * ((groups * n + 255) / 256)) / TT;
+    if (n > 1) t += 6500 + state * (350 + 330 * ((groups * (n - 1) + 255) / 256)) / TT;
+    return t;
+  };
+  int64_t best = 1, best_t = cost(1) * 95 / 100;
+  const int64_t most = std::min(kScanMaxGroups / groups, units / kScanMinUnits);
+  for (int64_t n = 2; n <= most; ++n)
+    if (cost(n) < best_t) {
+      best_t = cost(n);
+      best = n;
+    }
+  if (best < 2) return;
+  *nch = (int32_t)best;
+  *Tu = (int32_t)(units / best);
+  *rem = (int32_t)(units % best);
 }
 
 bool scan_supported(const ScanLaunch &a, const char **why) {
@@ -639,7 +670,7 @@ hipError_t launch_selective_scan(const ScanLaunch &L, hipStream_t s) {
   a.vec = (L.seq_len % 2 == 0) && al4(L.u) && al4(L.delta_raw) && al4(L.B) && al4(L.C) &&
           al4(L.y) && (!L.z || al4(L.z));
   const int64_t groups = (L.dim + SCH - 1) / SCH * L.batch;
-  scan_chunking(L.batch, L.dim, L.seq_len, a.vec != 0, &a.Tu, &a.rem, &a.nch);
+  scan_chunking(L.batch, L.dim, L.seq_len, &a.Tu, &a.rem, &a.nch);
   const bool sp = L.delta_softplus != 0, gate = L.z != nullptr;
   // the output kernel for this mode and these options
   auto out = [&](auto mode, unsigned grid) {
@@ -657,10 +688,9 @@ hipError_t launch_selective_scan(const ScanLaunch &L, hipStream_t s) {
     return hipGetLastError();
   }
   const dim3 sgrid((unsigned)(groups * (a.nch - 1)));
-  if (L.delta_softplus)
-    hipLaunchKernelGGL(selective_scan_state<true>, sgrid, dim3(NT), 0, s, a);
-  else
-    hipLaunchKernelGGL(selective_scan_state<false>, sgrid, dim3(NT), 0, s, a);
+  auto state = a.vec ? (sp ? selective_scan_state<true, true> : selective_scan_state<false, true>)
+                     : (sp ? selective_scan_state<true, false> : selective_scan_state<false, false>);
+  hipLaunchKernelGGL(state, sgrid, dim3(NT), 0, s, a);
   const int64_t lanes = L.batch * L.dim * ST;
   // a long chain of chunks: one wave per (batch, channel, state); up to 64
   // summaries the per-lane walk measured as fast or faster
