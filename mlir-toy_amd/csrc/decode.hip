@@ -8,10 +8,11 @@
 // exp2 domain:  M = max m_s, w_s = 2^(m_s - M), L = sum w_s l_s,
 // O = sum w_s o~_s / L, lse = (M + log2 L) ln 2.
 //
-// Work decomposition: one single-wave work-group per (batch, kv head,
-// split); the wave streams its split in 32-token steps through a private
-// LDS ring filled by global_load_lds_dwordx4 (no K/V byte passes through
-// VGPRs on its way to LDS). All query heads of the group
+// Work decomposition: one work-group per (batch, kv head, split), of a single
+// wave unless the launch is short of work-groups (decode_waves); a wave
+// streams its share of the split in 32-token steps through a private LDS ring
+// filled by global_load_lds_dwordx4 (no K/V byte passes through VGPRs on its
+// way to LDS). All query heads of the group
 // (heads_q / heads_kv <= 16) ride in one MFMA tile, so every K/V byte is
 // read from HBM exactly once. One wave per work-group lets the LDS budget,
 // not the work-group shape, set occupancy (measured fastest).
@@ -91,14 +92,14 @@ struct DecArgs {
   // fp8 scales: [B, Hk, nsb] per sb-token block; paged, [npages, Hk]
   const float *ksc, *vsc;
   float *part_o, *part_ml;
-  int32_t Hq, Hk, group, L, chunk, splits, nsb, sb;
+  int32_t B, Hq, Hk, group, L, chunk, splits, nsb, sb;
   float scale2;
   // paged KV (decode_partial_ring<true>, decode_partial_ring8<true>): token t
   // of sequence b lives in page btab[b * maxp + t / ps], at element offset
   // page * k_ps[0] + head * k_ps[1] + (t % ps) * tok (the same for V with
   // v_ps); seqlens[b] tokens
   const int32_t *btab, *seqlens;
-  int32_t ps, maxp, npages, tok;
+  int32_t ps, maxp, npages, tok, sorted, scaled;
   int64_t k_ps[2], v_ps[2];
 };
 
@@ -109,19 +110,58 @@ struct DecArgs {
 // share every token's row, and fp8 decode over such a pool measured 7%
 // faster (bf16 1%) with this order, while contiguous fp8 decode measured 1%
 // slower with it.
+//
+// Paged sequences have lengths of their own, and work-groups go round the
+// CUs in id order (measured: the k-th of an XCD to CU k % 32). a.sorted: they
+// are taken longest first, every other round of the GPU in reverse, so that a
+// CU's share of long and short ones adds up to nearly the same everywhere.
+// *Lb is the item's length.
 template <bool PAGED>
-__device__ inline void grid_item(const DecArgs &a, int id, int *b, int *hk, int *split) {
+__device__ inline void grid_item(const DecArgs &a, int id, int lane, int *b, int *hk, int *split,
+                                 int *Lb) {
   if (PAGED) {
     *hk = id % a.Hk;
     const int rest = id / a.Hk;
     *split = rest % a.splits;
-    *b = rest / a.splits;
+    int r = rest / a.splits;
+    if (!a.sorted) {
+      *b = r;
+      *Lb = min(max(a.seqlens[r], 0), a.L);  // out-of-range lengths are clamped
+      return;
+    }
+    const int per = 256 / (a.Hk * a.splits);  // sequences per round of the GPU
+    if (per > 1) {
+      const int j = r / per, n = min(per, a.B - j * per);
+      if (j & 1) r = j * per + n - 1 - (r - j * per);
+    }
+    // lane i's key orders sequence i: longest first, then by index
+    const int key = lane < a.B ? min(max(a.seqlens[lane], 0), a.L) * 64 + 63 - lane : -1;
+    int at = r;
+    if (!__all(lane >= a.B || key >> 6 == __builtin_amdgcn_readfirstlane(key) >> 6)) {
+      int rank = 0;
+      for (int i = 0; i < a.B; ++i) rank += __builtin_amdgcn_readlane(key, i) > key;
+      at = __builtin_ctzll(__ballot(lane < a.B && rank == r));
+    }
+    *b = at;
+    *Lb = __builtin_amdgcn_readlane(key, at) >> 6;
   } else {
     *split = id % a.splits;
     const int bk = id / a.splits;
     *b = bk / a.Hk;
     *hk = bk % a.Hk;
+    *Lb = a.L;
   }
+}
+
+// Tokens per split of a sequence of Lb tokens. a.scaled (paged): the split
+// count is the launch's, and a shorter sequence is cut into as many (smaller)
+// splits, so that every work-group has its share instead of the later ones
+// none; at the full length this is the launch's chunk.
+template <bool PAGED>
+__device__ inline int seq_chunk(const DecArgs &a, int Lb) {
+  if (!PAGED || !a.scaled) return a.chunk;
+  const int per = (Lb + a.splits - 1) / a.splits;
+  return max((per + 63) / 64 * 64, 64);
 }
 
 // bf16 bits of 4 E4M3 codes packed in one dword -> two dwords of bf16 pairs
@@ -147,27 +187,25 @@ constexpr int RSTEP = 32;                   // tokens per step
 constexpr int RTILE = RSTEP * DH * 2;       // bytes of one K or V tile
 constexpr int RSLOT = 2 * RTILE;            // K + V
 constexpr int RWAVE = 2 * RSLOT;            // two slots per wave
-constexpr int RW = 1;                       // waves per work-group (LDS-bound occupancy)
-constexpr int RT = 64 * RW;                 // threads per work-group
-constexpr int RLDS = RW * RWAVE;
 
-template <bool PAGED>
-__global__ __launch_bounds__(RT) void decode_partial_ring(DecArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+// RW: waves per work-group, each streaming its share of the split's tokens
+template <bool PAGED, int RW>
+__global__ __launch_bounds__(64 * RW) void decode_partial_ring(DecArgs a) {
+  constexpr int RT = 64 * RW;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[RW * RWAVE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, G = lane >> 4;  // MFMA column (query head) / lane group
   const int id = blockIdx.x;
-  int split, b, hk;
-  grid_item<PAGED>(a, id, &b, &hk, &split);
+  int split, b, hk, Lb;
+  grid_item<PAGED>(a, id, lane, &b, &hk, &split, &Lb);
   const int bk = b * a.Hk + hk;  // batch * Hk + kv head
   const int Gq = a.group;
-  // this sequence's length (paged: its own; out-of-range values clamped)
-  const int Lb = PAGED ? min(max(a.seqlens[b], 0), a.L) : a.L;
 
-  const int c0 = split * a.chunk;
-  const int c1 = min(c0 + a.chunk, Lb);
-  const int wlen = ((a.chunk + RW * RSTEP - 1) / (RW * RSTEP)) * RSTEP;
+  const int chunk = seq_chunk<PAGED>(a, Lb);
+  const int c0 = split * chunk;
+  const int c1 = min(c0 + chunk, Lb);
+  const int wlen = ((chunk + RW * RSTEP - 1) / (RW * RSTEP)) * RSTEP;
   const int t0 = c0 + w * wlen;
   const int t1 = min(t0 + wlen, c1);
   const int nsteps = t1 > t0 ? (t1 - t0 + RSTEP - 1) / RSTEP : 0;
@@ -401,12 +439,9 @@ __global__ __launch_bounds__(RT) void decode_partial_ring(DecArgs a) {
 // issued after it as well. kload_wait() waits for a buffer and ties the
 // buffer's registers to that wait, so nothing reads them earlier
 // (tests/test_isa_hazards.py checks the compiled code for it).
-constexpr int R8W = 1;                      // waves per work-group (LDS-bound occupancy)
-constexpr int R8T = 64 * R8W;
 constexpr int R8TILE = RSTEP * DH;          // bytes of one V code tile
 constexpr int R8P = 4;                      // steps in flight (K buffers, V ring slots)
 constexpr int R8WAVE = R8P * R8TILE;
-constexpr int R8LDS = R8W * R8WAVE;
 
 typedef int v2i32 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
@@ -441,23 +476,23 @@ __device__ inline void kload_wait(u32x4 (&k)[4]) {
                : "memory");
 }
 
-template <bool PAGED>
-__global__ __launch_bounds__(R8T) void decode_partial_ring8(DecArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+template <bool PAGED, int R8W>
+__global__ __launch_bounds__(64 * R8W) void decode_partial_ring8(DecArgs a) {
+  constexpr int R8T = 64 * R8W;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[R8W * R8WAVE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, G = lane >> 4;
   const int id = blockIdx.x;
-  int split, b, hk;
-  grid_item<PAGED>(a, id, &b, &hk, &split);
+  int split, b, hk, Lb;
+  grid_item<PAGED>(a, id, lane, &b, &hk, &split, &Lb);
   const int bk = b * a.Hk + hk;  // batch * Hk + kv head
   const int Gq = a.group;
-  // this sequence's length (paged: its own; out-of-range values clamped)
-  const int Lb = PAGED ? min(max(a.seqlens[b], 0), a.L) : a.L;
 
-  const int c0 = split * a.chunk;
-  const int c1 = min(c0 + a.chunk, Lb);
-  const int wlen = ((a.chunk + R8W * RSTEP - 1) / (R8W * RSTEP)) * RSTEP;
+  const int chunk = seq_chunk<PAGED>(a, Lb);
+  const int c0 = split * chunk;
+  const int c1 = min(c0 + chunk, Lb);
+  const int wlen = ((chunk + R8W * RSTEP - 1) / (R8W * RSTEP)) * RSTEP;
   const int t0 = c0 + w * wlen;
   const int t1 = min(t0 + wlen, c1);
   const int nsteps = t1 > t0 ? (t1 - t0 + RSTEP - 1) / RSTEP : 0;
@@ -914,6 +949,19 @@ bool decode_supported(const DecodeLaunch &a, const char **why) {
   return true;
 }
 
+// Waves per work-group. A launch short of work-groups leaves CUs without loads
+// in flight, and a wave's serial steps set its time; its splits are then
+// shared by several waves (merged in LDS). Once every CU holds the four or five
+// single-wave work-groups its LDS fits, more waves only add merges. Measured
+// (us, 1 / 2 / 4 waves): bf16, 136 work-groups of 256 tokens (B1 32/8 heads
+// L4100) 10.7 / 8.5 / 7.9, 512 of them (B2 L8192) 16.0 / 15.1 / 17.4, 1024
+// (B1 L32768) 29.7 / 30.6 / 34.9; fp8, whose ring takes half the LDS, 512
+// 13.4 / 12.9 / 11.6, 1024 21.9 / 21.9 / 22.6.
+int decode_waves(int64_t groups, bool fp8) {
+  if (groups <= (fp8 ? 512 : 256)) return 4;
+  return groups <= 512 ? 2 : 1;
+}
+
 hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
   DecArgs a;
   a.q = (const uint16_t *)L.q;
@@ -923,6 +971,7 @@ hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
   a.vsc = L.v_scale;
   a.part_o = L.part_o;
   a.part_ml = L.part_ml;
+  a.B = (int32_t)L.batch;
   a.Hq = (int32_t)L.heads_q;
   a.Hk = (int32_t)L.heads_kv;
   a.group = (int32_t)(L.heads_q / L.heads_kv);
@@ -944,20 +993,30 @@ hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
   a.v_ps[0] = L.v_pstride[0];
   a.v_ps[1] = L.v_pstride[1];
   const int grid = (int)(L.batch * L.heads_kv * L.splits);
-  // Both rings fit the dynamic LDS every launch may use without a per-kernel
-  // attribute (which would have to be set on each device), so none is set.
-  static_assert(RLDS <= 48 * 1024 && R8LDS <= 48 * 1024, "decode ring past the default LDS limit");
-  if (L.kv_dtype == 3) {
-    if (paged)
-      hipLaunchKernelGGL(decode_partial_ring8<true>, dim3(grid), dim3(R8T), R8LDS, s, a);
-    else
-      hipLaunchKernelGGL(decode_partial_ring8<false>, dim3(grid), dim3(R8T), R8LDS, s, a);
-  } else {
-    if (paged)
-      hipLaunchKernelGGL(decode_partial_ring<true>, dim3(grid), dim3(RT), RLDS, s, a);
-    else
-      hipLaunchKernelGGL(decode_partial_ring<false>, dim3(grid), dim3(RT), RLDS, s, a);
-  }
+  // Balancing ragged paged sequences (grid_item, seq_chunk). Scaled splits pay
+  // where a work-group is long, or where the launch takes more than one round
+  // (five bf16 work-groups per CU); sorting, some 1 us of a launch's start,
+  // where it is long (one lane per sequence, its length and index in 32 bits).
+  // Measured (us, before / scaled / sorted too, lengths an eighth to all of
+  // L): fp8 B32 32/8 heads L8192 77.5 / 67.9 / 62.8, B64 L4096 77.5 / - /
+  // 63.5, token-major B29 L7497 81.2 / 74.0 / 69.7, bf16 B16 L16384 114 / - /
+  // 104, B8 L8192 (256-token work-groups, 2048 of them) 34.9 / 33.0 / 35.0;
+  // without either, bf16 B4 16/4 L20000 (1264 of 256 tokens) 28.2 / 29.6.
+  a.scaled = paged && (L.chunk >= 512 || grid > 1280);
+  a.sorted = paged && L.batch > 1 && L.batch <= 64 && L.chunk >= 512 && L.seq_kv < 1 << 25;
+  const int rw = decode_waves(grid, L.kv_dtype == 3);
+  auto partial = [&](auto RW) {
+    constexpr int W = decltype(RW)::value;
+    auto k = L.kv_dtype == 3 ? (paged ? decode_partial_ring8<true, W> : decode_partial_ring8<false, W>)
+                             : (paged ? decode_partial_ring<true, W> : decode_partial_ring<false, W>);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(64 * W), 0, s, a);
+  };
+  if (rw == 4)
+    partial(std::integral_constant<int, 4>{});
+  else if (rw == 2)
+    partial(std::integral_constant<int, 2>{});
+  else
+    partial(std::integral_constant<int, 1>{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(decode_combine, dim3((unsigned)(L.batch * L.heads_q)), dim3(DH),
