@@ -23,6 +23,7 @@
 //                              transpose reads, B = P^T from S^T)
 // K/V loads are non-temporal: each byte is used once, and the nt hint
 // measured ~10% more HBM bandwidth for this stream.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -766,28 +767,38 @@ __global__ __launch_bounds__(64 * R8W) void decode_partial_ring8(DecArgs a) {
 }
 
 // One work-group per (batch, query head): combine the splits' partials.
-// Every thread (one head_dim element) first issues the loads of its first
-// kCombinePre splits' o~, which do not depend on the weights, so their
-// latency overlaps that of the (m, l) reads. Wave 0 reads every split's
-// (m, l) (one lane per split), reduces M and L across the wave and leaves
-// the weights 2^(m_s - M) in LDS; then each thread sums its splits' o~ in
-// split order.
+// SG groups of 128 threads (one head_dim element each) share out the splits,
+// group sg taking sg, sg + SG, ..; every thread first issues the loads of its
+// first kCombinePre o~, which do not depend on the weights, so their latency
+// overlaps that of the (m, l) reads. Wave 0 reads every split's (m, l) (one
+// lane per split), reduces M and L across the wave and leaves the weights
+// 2^(m_s - M) in LDS; each thread sums its splits' o~ in split order, and the
+// groups' sums meet in LDS (in place of the weights).
+//
+// Bound: a small kernel's launch (3-5 us) and, with one group, a dependent
+// round trip for every 8 splits past the first 16: SG keeps it to the first
+// loads up to 128 splits. Measured (us, the whole decode call, one group /
+// SG): 128 splits, B1 32/8 heads L32768 bf16 28.8 / 25.6, fp8 20.6 / 17.3; 125
+// splits, B1 8/1 L32000 fp8 14.4 / 9.9; 32 splits, B4 32/8 L8192 26.2 / 25.3.
 constexpr int kCombinePre = 16;
 
-__global__ __launch_bounds__(DH) void decode_combine(const float *part_o,
-                                                     const float *part_ml,
-                                                     uint16_t *o, float *lse,
-                                                     int32_t splits) {
-  extern __shared__ float wts[];  // [splits]
+template <int SG>
+__global__ __launch_bounds__(DH * SG) void decode_combine(const float *part_o,
+                                                          const float *part_ml, uint16_t *o,
+                                                          float *lse, int32_t splits) {
+  extern __shared__ float wts[];  // [max(splits, SG > 1 ? SG * DH : 0)]
   __shared__ float stat[2];
   const int64_t bh = blockIdx.x;
-  const int d = threadIdx.x;
+  const int d = threadIdx.x % DH, sg = threadIdx.x / DH;
   const float *ml = part_ml + bh * splits * 2;
   const float *po = part_o + bh * splits * DH + d;
   float pre[kCombinePre];
 #pragma unroll
-  for (int s = 0; s < kCombinePre; ++s) pre[s] = s < splits ? po[(int64_t)s * DH] : 0.0f;
-  if (d < 64) {
+  for (int i = 0; i < kCombinePre; ++i) {
+    const int s = sg + SG * i;
+    pre[i] = s < splits ? po[(int64_t)s * DH] : 0.0f;
+  }
+  if (threadIdx.x < 64) {
     float M = kNegFltMax;
     for (int s = d; s < splits; s += 64) M = fmaxf(M, ml[2 * s]);
 #pragma unroll
@@ -808,10 +819,18 @@ __global__ __launch_bounds__(DH) void decode_combine(const float *part_o,
   __syncthreads();
   float acc = 0.0f;
 #pragma unroll
-  for (int s = 0; s < kCombinePre; ++s)
-    if (s < splits) acc += wts[s] * pre[s];
+  for (int i = 0; i < kCombinePre; ++i)
+    if (sg + SG * i < splits) acc += wts[sg + SG * i] * pre[i];
 #pragma unroll 8
-  for (int s = kCombinePre; s < splits; ++s) acc += wts[s] * po[(int64_t)s * DH];
+  for (int s = sg + SG * kCombinePre; s < splits; s += SG) acc += wts[s] * po[(int64_t)s * DH];
+  if constexpr (SG > 1) {
+    __syncthreads();  // every weight has been read
+    wts[threadIdx.x] = acc;
+    __syncthreads();
+    if (sg > 0) return;
+#pragma unroll
+    for (int i = 1; i < SG; ++i) acc += wts[i * DH + d];
+  }
   const float Ls = stat[1];
   // an empty sequence (paged decode with length 0) has L = 0: O = 0, lse = -inf
   o[bh * DH + d] = Bf16Tag::from_f32(Ls > 0.0f ? acc / Ls : 0.0f);
@@ -1019,10 +1038,22 @@ hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
     partial(std::integral_constant<int, 1>{});
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(decode_combine, dim3((unsigned)(L.batch * L.heads_q)), dim3(DH),
-                     (size_t)L.splits * sizeof(float), s,
-                     (const float *)L.part_o, (const float *)L.part_ml, (uint16_t *)L.o,
-                     L.lse, (int32_t)L.splits);
+  auto combine = [&](auto G) {
+    constexpr int SG = decltype(G)::value;
+    const size_t lds = std::max<size_t>(L.splits, SG > 1 ? SG * DH : 0) * sizeof(float);
+    hipLaunchKernelGGL(decode_combine<SG>, dim3((unsigned)(L.batch * L.heads_q)), dim3(DH * SG),
+                       lds, s, (const float *)L.part_o, (const float *)L.part_ml,
+                       (uint16_t *)L.o, L.lse, (int32_t)L.splits);
+  };
+  // as many groups as keep a thread to its first loads
+  if (L.splits <= kCombinePre)
+    combine(std::integral_constant<int, 1>{});
+  else if (L.splits <= 2 * kCombinePre)
+    combine(std::integral_constant<int, 2>{});
+  else if (L.splits <= 4 * kCombinePre)
+    combine(std::integral_constant<int, 4>{});
+  else
+    combine(std::integral_constant<int, 8>{});
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-"""Decode launches short of work-groups (two or four waves share a split) and
-ragged paged batches (splits scaled to each sequence, sequences taken longest
+"""Decode launches short of work-groups (two or four waves share a split), the
+combine of many splits (groups of threads share them out) and ragged paged batches (splits scaled to each sequence, sequences taken longest
 first), at their edges against the oracle at the decode contract."""
 
 import numpy as np
@@ -48,6 +48,20 @@ def test_waves_per_split(B, Hq, Hk, L, splits, fp8):
         torch.cuda.synchronize()
         ro, rl, _ = oracle.decode_splitk(bits(q), bits(k), bits(v), oracle.BF16, num_splits=splits)
     _check(o, lse, ro, rl, fp8, "waves per split")
+
+
+@pytest.mark.parametrize("splits", [16, 17, 32, 33, 64, 65, 128, 129])
+def test_combine_thread_groups(splits):
+    """Split counts around those where the combine takes more thread groups,
+    every split one or two 64-token blocks."""
+    print(f"case: combine splits={splits}", flush=True)
+    L = splits * 64 - 5
+    q = randn((1, 8, 128), seed=8)
+    k, v = (randn((1, 2, L, 128), seed=s) for s in (9, 10))
+    o, lse = ops.decode_splitk(q.cuda(), k.cuda(), v.cuda(), num_splits=splits, return_lse=True)
+    torch.cuda.synchronize()
+    ro, rl, _ = oracle.decode_splitk(bits(q), bits(k), bits(v), oracle.BF16, num_splits=splits)
+    _check(o, lse, ro, rl, False, "combine thread groups")
 
 
 @pytest.mark.parametrize("fp8", [False, True])
