@@ -30,6 +30,7 @@ struct SplitArgs {
   int32_t nsplit;  // 0: the plain kernel; 1: no partials
   int32_t kbs;     // 64-key blocks per split
   int32_t packed;
+  int32_t halves;  // 2: eight waves, four on each half of the split's keys
   float *po;       // [B * Hq * Sq, nsplit, head_dim]
   float *pml;      // [B * Hq * Sq, nsplit, 2]: (m, l)
 };

@@ -385,6 +385,15 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
 //   / 27; 8 x 32/4 heads, 1 over 4000 68 / 17 / 16; head_dim 64, 1 x 16/4,
 //   250 over 8000 99 / 23.6 / 8. Where it stays whole: 1 x 32 heads, 1000 over
 //   1000 causal 22.8 / 30.1 with two splits; 1 x 32/8, 256 over 512 13.9 / 17.1.
+// - Halves: a launch of at most one work-group per CU that stays whole has
+//   eight waves per work-group, four on each half of the keys, merged in LDS.
+//   The waves of a SIMD run in step, so their matrix and vector work overlaps
+//   less than two work-groups' (1.75 us a block pair, 1.5 us for the merge;
+//   under splits it lost to more of them: 500 over 4000 56.7 / 45.5). Measured
+//   (us, four waves / eight): 1 x 16 heads causal S 1500 30.1 / 25.6, S 2000
+//   38.4 / 32.1, 1 x 32 S 1000 22.8 / 20.6, S 640 16.4 / 15.9, S 512 14.2 /
+//   14.2; head_dim 64 S 2000 29.0 / 22.8, 1 x 32 S 1000 17.0 / 14.5, S 512
+//   10.4 / 9.9.
 // - Without the mask the head_dim-128 kernel runs two query blocks per
 //   work-group; up to 512 blocks they are better apart (1 x 4 heads, 512
 //   over 512: 25.0 / 13.4).
@@ -406,24 +415,30 @@ AttnSplit attn_split(const AttnLaunch &L, bool partials) {
     int64_t t = (nkb + ns - 1) / ns * step;
     if (ns > 1) {
       // states written and read: causal blocks leave the splits past them empty
-      const int64_t states = causal ? ns - (ns - 1) * std::min(L.seq_q, L.seq_kv) / (2 * L.seq_kv) : ns;
-      t += 3000 + 4500 + rows * states * (L.head_dim + 2) * 8 / 5000;
+      const int64_t empty = causal ? (ns - 1) * std::min(L.seq_q, L.seq_kv) : 0;
+      t += 3000 + 4500 +
+           (int64_t)((double)rows * (L.head_dim + 2) * 8 / 5000 *
+                     (ns - (double)empty / (2.0 * L.seq_kv)));
     } else {
       t += 3000;
     }
     return t;
   };
   int64_t best = 1;
-  if (partials && wgs <= kSlots / 2) {
-    const int64_t one = cost(1) * 95 / 100;
-    int64_t best_t = one;
-    for (int64_t ns = 2; ns <= kMaxAttnSplits && wgs * ns <= kSlots && ns <= nkb; ++ns)
+  if (wgs <= kSlots / 2) {
+    if (nkb >= (d128 ? 10 : 8)) p.halves = 2;
+    const int64_t one =
+        p.halves == 2 ? std::min(cost(1), 4500 + (nkb + 1) / 2 * (d128 ? 1750 : 1150)) : cost(1);
+    int64_t best_t = one * 95 / 100;
+    for (int64_t ns = 2;
+         partials && ns <= kMaxAttnSplits && wgs * ns <= kSlots && ns <= nkb; ++ns)
       if (cost(ns) < best_t) {
         best_t = cost(ns);
         best = ns;
+        p.halves = 1;
       }
   }
-  if (best == 1 && !(p.packed && 2 * packed <= plain) &&
+  if (best == 1 && p.halves == 1 && !(p.packed && 2 * packed <= plain) &&
       !(d128 && !causal && wgs <= kSlots))
     return AttnSplit();
   p.kbs = (int32_t)((nkb + best - 1) / best);
@@ -469,6 +484,7 @@ hipError_t launch_attn_fwd(const AttnLaunch &L, const AttnSplit &split, void *wo
       x.nsplit = split.nsplit;
       x.kbs = split.kbs;
       x.packed = split.packed;
+      x.halves = split.halves;
       x.po = (float *)workspace;
       x.pml = x.po + (size_t)(L.batch * L.heads_q * L.seq_q) * split.nsplit * L.head_dim;
       return launch_attn_tile(a, x, L.dtype, (int)L.head_dim, causal, s);

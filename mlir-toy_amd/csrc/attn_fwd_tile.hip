@@ -30,28 +30,29 @@ namespace {
 
 // SPLIT: a work-group takes one split of the keys (x.kbs blocks) and, packed,
 // rows that run through the heads of its KV head; with more than one split
-// it leaves its unnormalised O and (m, l) for attn_combine. 208 registers at
-// head_dim 128 (two work-groups per CU). What it measured stands at
+// it leaves its unnormalised O and (m, l) for attn_combine. KW = 2: eight
+// waves, four on each half of the keys, whose states merge in LDS lane to lane.
+// 210 registers at head_dim 128 (two waves per SIMD). What it measured stands at
 // attn_split, which chooses the cut.
-template <class E, int HD, bool CAUSAL, bool SPLIT>
-__global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) {
+template <class E, int HD, bool CAUSAL, bool SPLIT, int KW>
+__global__ __launch_bounds__(NT * KW, 2 / KW) void attn_fwd_tile(AttnArgs a, SplitArgs x) {
   typedef typename E::vec8 V8;
   constexpr int TILE = TileLoader<HD>::TILE_BYTES;
   constexpr int ROWB = HD * 2;   // bytes per LDS row
   constexpr int NST = HD / 16;   // QK^T k-steps
   constexpr int NB = HD / 32;    // 32-wide head_dim blocks of O^T
   constexpr int NQK = 2 * NST, NPV = 4 * NB;  // MFMAs per key block
-  // K slots 0 and 1, then V slots 0 and 1; block t uses slot t & 1
-  __shared__ __attribute__((aligned(16))) uint8_t smem[4 * TILE];
-  const uint8_t *const kt0 = smem;
-  const uint8_t *const vt0 = smem + 2 * TILE;
-  auto kslot = [&](int t) { return kt0 + (t & 1) * TILE; };
-  auto vslot = [&](int t) { return vt0 + (t & 1) * TILE; };
-
+  // per key half: K slots 0 and 1, then V slots 0 and 1; block t uses slot t & 1
+  __shared__ __attribute__((aligned(16))) uint8_t smem[KW * 4 * TILE];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = KW > 1 ? wave & 3 : wave, half = KW > 1 ? wave >> 2 : 0;
   const int lq = lane & 31, g = lane >> 5;
+  const uint8_t *const kt0 = smem + half * 4 * TILE;
+  const uint8_t *const vt0 = kt0 + 2 * TILE;
+  auto kslot = [&](int t) { return kt0 + (t & 1) * TILE; };
+  auto vslot = [&](int t) { return vt0 + (t & 1) * TILE; };
 
   // Work-group -> (kv head, split, query head of its group, query block): kv
   // heads fastest, so that (with a multiple of 8 of them) id % 8, the XCD,
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) 
   };
   // key blocks kb0 .. kb0 + nv - 1 of the work-group, the first nkw of them
   // this wave's
-  const int kb0 = SPLIT ? split * x.kbs : 0;
+  int kb0 = SPLIT ? split * x.kbs : 0;
   int nv = (a.Sk + BN - 1) / BN, nkw = nv, lo_w = 0;
   if (CAUSAL) {
     int lo, hi;
@@ -108,8 +109,19 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) 
     nv = min(max(nv - kb0, 0), x.kbs);
     nkw = min(max(nkw - kb0, 0), x.kbs);
   }
+  // the trips of the key loop: with two halves, the first takes the odd block
+  int trips = nv;
+  if constexpr (KW > 1) {
+    trips = (nv + 1) >> 1;
+    const int first = half ? trips : 0, n = half ? nv - trips : trips;
+    kb0 += first;
+    nv = n;
+    nkw = min(max(nkw - first, 0), n);
+  }
   nv = __builtin_amdgcn_readfirstlane(nv);
   nkw = __builtin_amdgcn_readfirstlane(nkw);
+  trips = KW > 1 ? __builtin_amdgcn_readfirstlane(trips) : nv;
+  if constexpr (SPLIT) kb0 = __builtin_amdgcn_readfirstlane(kb0);
 
   const TileLoader<HD> kl = make_loader<HD, false>(kp, a.ks2, w, lane);
   const TileLoader<HD> vl = make_loader<HD, true>(vp, a.vs2, w, lane);
@@ -184,7 +196,7 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) 
   if (nkw > 0) qk_from(kslot(0), k_operand(kslot(0), 0), k_operand(kslot(0), 1));
   __syncthreads();  // every wave is done with K slot 0 before it is refilled
 
-  for (int jb = 0; jb < nv; ++jb) {
+  for (int jb = 0; jb < trips; ++jb) {
     // K of block jb + 2 goes to the slot block jb's K has left, V of block
     // jb + 1 to the slot of block jb - 1's V
     if (jb + 2 < nv) load_k(jb + 2);
@@ -280,13 +292,41 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_tile(AttnArgs a, SplitArgs x) 
     __syncthreads();
   }
 
-  const float ltot = pair_sum(lsum);
+  float ltot = pair_sum(lsum);
+  if constexpr (KW > 1) {
+    // the second half's state to its row's wave of the first, lane to lane,
+    // through the K/V slots (free since the loop's last barrier)
+    f32x4 *const box = (f32x4 *)smem + (w * (4 * NB) * 64 + lane);
+    f32x2 *const mlbox = (f32x2 *)(smem + KW * 4 * TILE) - 4 * 64 + (w * 64 + lane);
+    if (half) {
+#pragma unroll
+      for (int v = 0; v < 4 * NB; ++v)
+        box[v * 64] = f32x4{o[v >> 2][4 * (v & 3)], o[v >> 2][4 * (v & 3) + 1],
+                            o[v >> 2][4 * (v & 3) + 2], o[v >> 2][4 * (v & 3) + 3]};
+      *mlbox = f32x2{m, ltot};
+    }
+    __syncthreads();
+    if (half) return;
+    const f32x2 ml = *mlbox;
+    const float M = fmaxf(m, ml[0]), w0 = fast_exp2(m - M), w1 = fast_exp2(ml[0] - M);
+    ltot = ltot * w0 + ml[1] * w1;
+    m = M;
+#pragma unroll
+    for (int v = 0; v < 4 * NB; ++v) {
+      const f32x4 other = box[v * 64];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = 4 * (v & 3) + r;
+        o[v >> 2][e] = fmaf(o[v >> 2][e], w0, other[r] * w1);
+      }
+    }
+  }
   if (row < rows) {
     const int64_t grow = ((int64_t)b * a.Hq + h0 + hr) * a.Sq + pos;  // row of [B, Hq, Sq]
     if constexpr (SPLIT) {
       if (x.nsplit > 1) {  // this split's state, for attn_combine
         const int64_t part = grow * x.nsplit + split;
-        if (nv > 0) {
+        if (trips > 0) {
           float *op = x.po + part * HD + 4 * g;
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb)
@@ -382,7 +422,11 @@ void launch_split(AttnArgs a, const SplitArgs &x, hipStream_t s) {
   const int rows = x.packed ? a.group * a.Sq : a.Sq;
   a.nqb = (rows + BM - 1) / BM;
   const unsigned grid = (unsigned)a.nqb * (x.packed ? BHk : a.BH) * x.nsplit;
-  hipLaunchKernelGGL((attn_fwd_tile<E, HD, CAUSAL, true>), dim3(grid), dim3(NT), 0, s, a, x);
+  if (x.halves > 1)
+    hipLaunchKernelGGL((attn_fwd_tile<E, HD, CAUSAL, true, 2>), dim3(grid), dim3(2 * NT), 0, s, a,
+                       x);
+  else
+    hipLaunchKernelGGL((attn_fwd_tile<E, HD, CAUSAL, true, 1>), dim3(grid), dim3(NT), 0, s, a, x);
   if (x.nsplit > 1) {
     const int64_t nrows = (int64_t)a.BH * a.Sq, per = NT / (HD / 4);
     auto k = x.nsplit <= 4    ? attn_combine<E, HD, 4>
@@ -404,9 +448,9 @@ void launch_e(const AttnArgs &a, const SplitArgs &x, int head_dim, bool causal, 
   }
   const dim3 grid((unsigned)(a.nqb * a.BH));
   if (causal)
-    hipLaunchKernelGGL((attn_fwd_tile<E, 64, true, false>), grid, dim3(NT), 0, s, a, x);
+    hipLaunchKernelGGL((attn_fwd_tile<E, 64, true, false, 1>), grid, dim3(NT), 0, s, a, x);
   else
-    hipLaunchKernelGGL((attn_fwd_tile<E, 64, false, false>), grid, dim3(NT), 0, s, a, x);
+    hipLaunchKernelGGL((attn_fwd_tile<E, 64, false, false, 1>), grid, dim3(NT), 0, s, a, x);
 }
 
 }  // namespace

@@ -25,6 +25,7 @@ struct AttnLaunch {
 struct AttnSplit {
   int32_t nsplit = 0;  // key splits (1: none, the rows are packed only)
   int32_t kbs = 0;     // 64-key blocks per split
+  int32_t halves = 1;  // 2: eight waves, four on each half of the keys
   int32_t packed = 0;  // the query heads of a KV head form one run of rows
   size_t bytes = 0;    // workspace the splits' states take
 };
