@@ -44,7 +44,10 @@ namespace {
 // in a lane): B2 H12 S1500 D64 causal 361 -> 81 us (85 TFLOP/s; a large fp32
 // GEMM reaches 154 on this card), B2 H16 S1024 D128 1434 -> 162 us (106
 // TFLOP/s), B1 H1 S128 D64 10.3 -> 4.9 us (three quarters of it launch
-// latency).
+// latency). Reading K and V by ranges (f32_rows) took the 64-bit address of
+// every row, 15 quarter-rate multiplies per 16 keys, out of the loop: the first
+// two 81 -> 78 and 164 -> 148 us, B4 H16 S800 D32 61.7 -> 55.3, one query over
+// 2048 keys of 8 heads, D128, 49.3 -> 39.4.
 constexpr int F32_KB = 16;  // keys per block and wave
 // The split of the work by the number of 32-row blocks of the launch. Below
 // the line the GPU is short of work-groups and a wave's serial key loop sets
@@ -74,8 +77,19 @@ __device__ inline typename F32Vec<N>::type load_f32(const float *p) {
   return v;
 }
 
+// The rows row0 .. row0 + F32_KB - 1 of one head's K or V (seq rows, stride
+// floats apart), to the end of the last one that exists: rows beyond it start at
+// or past the range's end (stride >= D), where loads return 0.
+__device__ inline __amdgpu_buffer_rsrc_t f32_rows(const float *head, int64_t stride, int row0,
+                                                  int seq, int D) {
+  const int n = max(min(seq - row0, F32_KB), 0);
+  const int bytes = max(4 * ((n - 1) * (int)stride + D), 0);  // n = 0: stride >= D
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(head + row0 * stride), (short)0,
+                                           bytes, 0x00020000);
+}
+
 // VEC: 16-byte loads and stores (every base and stride a multiple of 16
-// bytes); otherwise one element each
+// bytes, and K and V rows as f32_rows addresses them); otherwise one element each
 template <int D, bool CAUSAL, int NQ, int NW, bool VEC>
 __global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
   constexpr int NM = D / 16;             // 16-wide head_dim blocks
@@ -106,13 +120,24 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
     nkb = min(nkb, last < 0 ? 0 : last / F32_KB + 1);
   }
 
-  // rows and keys past the end read the last one (rows are not stored, keys
-  // are masked), so no load is guarded
+  // VEC: a block's rows are read through a buffer resource that begins with the
+  // block and ends with the tensor's last row, so a lane's offsets are fixed
+  // and rows past the end read 0. Otherwise rows past the end read the last
+  // one. Either way no load is guarded, and such keys are masked.
+  const int krow = i * (int)a.ks2 + 4 * g, vcol = VW * i, vrow = (int)a.vs2;
   f32x4 kf[NM];
   auto load_k = [&](int kb) {
-    const float *r = kp + min(kb * F32_KB + i, a.Sk - 1) * a.ks2 + 4 * g;
+    if constexpr (VEC) {
+      const auto r = f32_rows(kp, a.ks2, kb * F32_KB, a.Sk, D);
 #pragma unroll
-    for (int m = 0; m < NM; ++m) kf[m] = load_f32<4, VEC>(r + 16 * m);
+      for (int m = 0; m < NM; ++m)
+        kf[m] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 4 * krow + 64 * m, 0, 0));
+    } else {
+      const float *r = kp + min(kb * F32_KB + i, a.Sk - 1) * a.ks2 + 4 * g;
+#pragma unroll
+      for (int m = 0; m < NM; ++m) kf[m] = load_f32<4, VEC>(r + 16 * m);
+    }
   };
   load_k(w);
   f32x4 qf[NQ][NM];
@@ -139,11 +164,25 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
   for (int kb = w; kb < nkb; kb += NW) {
     const int key0 = kb * F32_KB;
     VV vf[4][VL];  // V of keys 4 g + r
+    if constexpr (VEC) {
+      const auto rows = f32_rows(vp, a.vs2, key0, a.Sk, D);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float *vr = vp + min(key0 + 4 * g + r, a.Sk - 1) * a.vs2 + VW * i;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int c = 0; c < VL; ++c) vf[r][c] = load_f32<VW, VEC>(vr + 64 * c);
+        for (int c = 0; c < VL; ++c) {
+          const int at = 4 * ((4 * g + r) * vrow + vcol) + 256 * c;
+          if constexpr (VW == 4)
+            vf[r][c] = __builtin_bit_cast(VV, __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0));
+          else
+            vf[r][c] = __builtin_bit_cast(VV, __builtin_amdgcn_raw_buffer_load_b64(rows, at, 0, 0));
+        }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float *vr = vp + min(key0 + 4 * g + r, a.Sk - 1) * a.vs2 + VW * i;
+#pragma unroll
+        for (int c = 0; c < VL; ++c) vf[r][c] = load_f32<VW, VEC>(vr + 64 * c);
+      }
     }
     // two chains of D / 2 terms per score: half the rounding of one chain of D,
     // and no product waits for the one just before it
@@ -471,6 +510,9 @@ hipError_t launch_attn_fwd(const AttnLaunch &L, const AttnSplit &split, void *wo
     bool vec = true;
     for (int i = 0; i < 3; ++i)
       vec = vec && L.qs[i] % 4 == 0 && L.ks[i] % 4 == 0 && L.vs[i] % 4 == 0 && L.os[i] % 4 == 0;
+    // f32_rows: rows that do not overlap (one past the end would start inside
+    // the range), a block's offsets in 31 bits
+    for (int64_t st : {L.ks[2], L.vs[2]}) vec = vec && st >= L.head_dim && st < (1 << 25);
     for (const void *p : {L.q, L.k, L.v, (const void *)L.o}) vec = vec && ((uintptr_t)p & 15u) == 0;
     switch (L.head_dim) {
       case 32: launch_f32<32>(a, causal, vec, s); break;
