@@ -417,12 +417,13 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
 //   one work-group per CU the chain is cut. The count is the one with the
 //   least estimated time, from what the kernels measured: a key block takes
 //   1.05 us alone on a CU and 1.65 us beside another work-group (head_dim 64:
-//   0.75 and 1.1), a launch 3 us, the combine 4.5 us, and the states
+//   0.94 and 1.35), a launch 3 us, the combine 4.5 us, and the states
 //   move at 5 TB/s. A cut has to promise 5%. Measured (us, one piece /
 //   chosen cut / its count): 1 x 32/8 heads, 250 queries over 8000 keys 134 /
 //   44.5 / 8; 500 over 4000 71 / 44 / 4; 1 x 8 heads, 128 over 12000 197 / 22
 //   / 27; 8 x 32/4 heads, 1 over 4000 68 / 17 / 16; head_dim 64, 1 x 16/4,
-//   250 over 8000 99 / 23.6 / 8. Where it stays whole: 1 x 32 heads, 1000 over
+//   250 over 8000 125 / 28.4 / 8; 1 x 4, 2048 over 2048 causal 35.9 / 18.7 / 4;
+//   3 x 4, 2 over 430 9.6 / 6.8 / 7. Where it stays whole: 1 x 32 heads, 1000 over
 //   1000 causal 22.8 / 30.1 with two splits; 1 x 32/8, 256 over 512 13.9 / 17.1.
 // - Halves: a launch of at most one work-group per CU that stays whole has
 //   eight waves per work-group, four on each half of the keys, merged in LDS.
@@ -431,8 +432,8 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
 //   under splits it lost to more of them: 500 over 4000 56.7 / 45.5). Measured
 //   (us, four waves / eight): 1 x 16 heads causal S 1500 30.1 / 25.6, S 2000
 //   38.4 / 32.1, 1 x 32 S 1000 22.8 / 20.6, S 640 16.4 / 15.9, S 512 14.2 /
-//   14.2; head_dim 64 S 2000 29.0 / 22.8, 1 x 32 S 1000 17.0 / 14.5, S 512
-//   10.4 / 9.9.
+//   14.2; head_dim 64 (1.3 us a pair) S 2000 35.5 / 28.2, 1 x 32 S 1000 20.8 /
+//   17.7, S 512 12.7 / 11.8.
 // - Without the mask the head_dim-128 kernel runs two query blocks per
 //   work-group; up to 512 blocks they are better apart (1 x 4 heads, 512
 //   over 512: 25.0 / 13.4).
@@ -450,7 +451,7 @@ AttnSplit attn_split(const AttnLaunch &L, bool partials) {
   const int64_t wgs = p.packed ? packed : plain;
   // estimated nanoseconds with the keys cut into ns splits
   auto cost = [&](int64_t ns) {
-    const int64_t step = wgs * ns <= kSlots / 2 ? (d128 ? 1050 : 750) : (d128 ? 1650 : 1100);
+    const int64_t step = wgs * ns <= kSlots / 2 ? (d128 ? 1050 : 940) : (d128 ? 1650 : 1350);
     int64_t t = (nkb + ns - 1) / ns * step;
     if (ns > 1) {
       // states written and read: causal blocks leave the splits past them empty
@@ -467,7 +468,7 @@ AttnSplit attn_split(const AttnLaunch &L, bool partials) {
   if (wgs <= kSlots / 2) {
     if (nkb >= (d128 ? 10 : 8)) p.halves = 2;
     const int64_t one =
-        p.halves == 2 ? std::min(cost(1), 4500 + (nkb + 1) / 2 * (d128 ? 1750 : 1150)) : cost(1);
+        p.halves == 2 ? std::min(cost(1), 4500 + (nkb + 1) / 2 * (d128 ? 1750 : 1300)) : cost(1);
     int64_t best_t = one * 95 / 100;
     for (int64_t ns = 2;
          partials && ns <= kMaxAttnSplits && wgs * ns <= kSlots && ns <= nkb; ++ns)

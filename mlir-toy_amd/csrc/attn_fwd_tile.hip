@@ -7,20 +7,23 @@
 // global_load_lds_dwordx4 into two slots per operand, the transposed products
 //   S^T = K . Q^T   (A = K rows from LDS, B = Q^T in VGPRs)
 //   O^T = V^T . P^T (A = V^T from LDS via ds_read_b64_tr_b16, B = P^T)
-// on v_mfma_f32_32x32x16 (one query row per lane), block j+1's QK^T in the
-// MFMA stream of block j's P.V, and the lazily moved running max.
+// on v_mfma_f32_32x32x16 (one query row per lane), and block j+1's QK^T in the
+// MFMA stream of block j's P.V. At head_dim 128 the running max moves lazily,
+// as in that kernel; at head_dim 64 it moves with every block that passes it,
+// so that a row's largest p is 1 and takes no rounding to 16 bits.
 //
-// Bound: at head_dim 64 a key block's softmax (128 vector instructions a
-// wave, about 640 cycles) outweighs its 16 MFMAs (512 cycles); counters show
-// the two units busy in 87% of the cycles, half of the matrix time under
-// vector work. Two work-groups per CU (182 registers). Three or four of them
-// (127 registers, with the copies' rare tail computed in place) measured the
-// same within 3%, and a barrier for every second key block (four slots per
-// operand) 8% slower, so neither occupancy nor the barrier holds it back.
-// Measured (GPU time, against a kernel that staged K and V through registers
-// and transposed V while writing it to LDS): B4 H16 S2048 causal 58.5 -> 43-45
-// us (770 TFLOP/s), without the mask 105 -> 73-75 us (930), B1 H8 S4096 causal
-// 83 -> 52 us, B4 H8 S55 5.1 -> 4.0 us.
+// Bound: at head_dim 64 a key block's softmax (about 190 vector instructions a
+// wave with the rescale of O) outweighs its 16 MFMAs (512 cycles). Two
+// work-groups per CU (162-168 registers). Measured on the lazy form, three or
+// four of them (127 registers, with the copies' rare tail computed in place)
+// came within 3%, and a barrier for every second key block (four slots per
+// operand) was 8% slower, so neither occupancy nor the barrier holds it back.
+// Measured (GPU time, graph replays, against a kernel that staged K and V
+// through registers and transposed V while writing it to LDS): B4 H16 S2048
+// causal 64 -> 54.5 us (630 TFLOP/s), without the mask 105.6 -> 90.3 (760), B1
+// H8 S4096 causal 83.5 -> 50.4, B4 H8 S55 5.35 -> 4.5. A lazy max here measured
+// 51, 77.8, 41.2 and 4.3 us and 3-6% more error against 64 bits (f16, N(0, 1)),
+// so it is not used.
 #include "attn_args.h"
 #include "attn_tile.h"
 #include "kernels.h"
@@ -235,15 +238,7 @@ __global__ __launch_bounds__(NT * KW, 2 / KW) void attn_fwd_tile(AttnArgs a, Spl
           }
         }
       };
-      // the block max is only formed when it can matter (see the head_dim-128
-      // kernel): past the first key block, a lane sum of at most 2^kSlack
-      // bounds every p by it, and m keeps
-      bool full = jb == 0;
-      if (!full) {
-        expo();
-        full = __any(!(rs <= kSumCap));
-      }
-      if (full) {
+      auto raise_max = [&](float slack) {  // m to the block's max where that passes m + slack
         float mx = -INFINITY;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -251,7 +246,7 @@ __global__ __launch_bounds__(NT * KW, 2 / KW) void attn_fwd_tile(AttnArgs a, Spl
           for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
         mx = pair_max(mx);
         const float m_blk = mx * sc;
-        if (__any(m_blk > m + kSlack)) {
+        if (__any(m_blk > m + slack)) {
           const float m_new = fmaxf(m, m_blk);
           const float alpha = fast_exp2(m - m_new);
           lsum *= alpha;
@@ -261,7 +256,25 @@ __global__ __launch_bounds__(NT * KW, 2 / KW) void attn_fwd_tile(AttnArgs a, Spl
             for (int r = 0; r < 16; ++r) o[nb][r] *= alpha;
           m = m_new;
         }
+      };
+      if constexpr (HD == 64) {
+        // the max of every block: a row's largest p is then exactly 1, with no
+        // rounding to 16 bits
+        raise_max(0.0f);
         expo();
+      } else {
+        // the block max is only formed when it can matter (see the head_dim-128
+        // kernel): past the first key block, a lane sum of at most 2^kSlack
+        // bounds every p by it, and m keeps
+        bool full = jb == 0;
+        if (!full) {
+          expo();
+          full = __any(!(rs <= kSumCap));
+        }
+        if (full) {
+          raise_max(kSlack);
+          expo();
+        }
       }
       lsum += rs;
 
