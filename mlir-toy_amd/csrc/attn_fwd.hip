@@ -49,6 +49,16 @@ namespace {
 // two 81 -> 78 and 164 -> 148 us, B4 H16 S800 D32 61.7 -> 55.3, one query over
 // 2048 keys of 8 heads, D128, 49.3 -> 39.4.
 constexpr int F32_KB = 16;  // keys per block and wave
+// A wave adds up P.V over F32_STRETCH blocks, then adds that to the sum of its
+// earlier stretches, kept in LDS: the rounding of a sum of n terms grows with
+// sqrt(n), and 96 terms at a time keep it below that of the vector-ALU kernel,
+// which summed Sk / 16 terms in each of 16 lanes. Relative error against 64
+// bits (1e-7; N(0, 1), no mask; that kernel / one sum per wave / stretches): S
+// 2048 D32 3.25 / 4.47 / 2.56, D64 3.75 / 4.58 / 2.76, D128 4.62 / 4.81 / 3.15; S
+// 512 D32 2.52 / 2.59 / 2.29. The stretches cost up to 4% of the time (B2 H12
+// S1500 D64 causal 75.0 -> 78.1 us, the figures above being without them; D128
+// no mask and D32 1%); four blocks instead of six cost 1% more.
+constexpr int F32_STRETCH = 6;
 // The split of the work by the number of 32-row blocks of the launch. Below
 // the line the GPU is short of work-groups and a wave's serial key loop sets
 // the time, so 16-row work-groups cut the keys eight ways; above it the
@@ -89,9 +99,12 @@ __device__ inline __amdgpu_buffer_rsrc_t f32_rows(const float *head, int64_t str
 }
 
 // VEC: 16-byte loads and stores (every base and stride a multiple of 16
-// bytes, and K and V rows as f32_rows addresses them); otherwise one element each
+// bytes, and K and V rows as f32_rows addresses them); otherwise one element
+// each. At head_dim 32 the causal form is held to five waves per SIMD (left to
+// itself it takes 98 registers, two too many: B4 H16 S800 33.3 / 30.3 us)
 template <int D, bool CAUSAL, int NQ, int NW, bool VEC>
-__global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
+__global__ __launch_bounds__(64 * NW, D == 32 && CAUSAL && NQ == 2 ? 5 : 1) void attn_fwd_f32(
+    AttnArgs a) {
   constexpr int NM = D / 16;             // 16-wide head_dim blocks
   constexpr int VW = NM < 4 ? NM : 4;    // head_dim elements per V load
   constexpr int VL = NM / VW;            // V loads per key
@@ -160,6 +173,21 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
     for (int c = 0; c < NM; ++c) o[n][c] = f32x4{0, 0, 0, 0};
   }
   const float sc = a.scale2;
+
+  // the sums of the earlier stretches, in this wave's part of mo (value v of the
+  // lane at 64 v), scaled by the max of their last block (in its part of mm)
+  int since = 0;  // blocks since the last stretch ended
+  bool banked = false;
+  auto bank = [&](int v) { return (f32x4 *)&mo[w][0][0] + 64 * v + lane; };
+  auto add_bank = [&](int n) {
+    const float keep = fast_exp2(mm[w][16 * n + i] - m[n]);
+#pragma unroll
+    for (int c = 0; c < NM; ++c) {
+      const f32x4 old = *bank(n * NM + c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[n][c][r] = fmaf(old[r], keep, o[n][c][r]);
+    }
+  };
 
   for (int kb = w; kb < nkb; kb += NW) {
     const int key0 = kb * F32_KB;
@@ -257,7 +285,24 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_f32(AttnArgs a) {
         for (int n = 0; n < NQ; ++n)
           o[n][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][c / VW][c % VW], s[n][r], o[n][c],
                                                          0, 0, 0);
+    if (++since == F32_STRETCH) {
+      since = 0;
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        if (banked) add_bank(n);
+        mm[w][16 * n + i] = m[n];
+#pragma unroll
+        for (int c = 0; c < NM; ++c) {
+          *bank(n * NM + c) = o[n][c];
+          o[n][c] = f32x4{0, 0, 0, 0};
+        }
+      }
+      banked = true;
+    }
   }
+  if (banked)
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) add_bank(n);
 
   // merge the waves' states
 #pragma unroll

@@ -59,3 +59,23 @@ def test_d64_rounds_no_more_than_the_tile_program(B, H, S, causal, dtype):
     e, limit = _rel(got, exact), _rel(rounded, exact)
     print(f"  error against 64 bits {e:.4e}, the tile program's {limit:.4e}", flush=True)
     assert e <= 1.01 * limit
+
+
+@pytest.mark.parametrize("B,H,D", [(2, 4, 32), (2, 4, 64), (1, 1, 32)])
+def test_fp32_sums_stay_short(B, H, D):
+    """fp32 over 2048 keys, no mask: four waves a row block (eight with one
+    head), so 512 (256) keys a wave. A sum of n rounded additions whose partial
+    sums grow as a random walk is off by u sqrt(n / 2), u = 2^-23 / sqrt(12) *
+    0.74 (a half ulp's spread over a binade). Beyond the error at 128 keys (a
+    block or two a wave) the long rows may show that of n = 128 terms, plus 10%."""
+    from neptune_hip import ops
+    print(f"case: fp32 sums B={B} H={H} D={D}", flush=True)
+    q, k, v = (randn((B, H, 2048, D), seed=s, dtype=torch.float32).cuda() for s in (4, 5, 6))
+    err = {}
+    for n in (128, 2048):
+        kn, vn = k[:, :, :n].contiguous(), v[:, :, :n].contiguous()
+        exact, _ = _exact_and_htile(q, kn, vn, False)
+        err[n] = _rel(ops.attention(q, kn, vn), exact)
+    chain = 2.0 ** -23 / math.sqrt(12) * 0.74 * math.sqrt(128 / 2)
+    print(f"  error against 64 bits {err}, sums of 128 terms {chain:.2e}", flush=True)
+    assert err[2048] <= 1.1 * math.hypot(err[128], chain)
