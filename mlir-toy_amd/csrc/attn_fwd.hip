@@ -366,8 +366,7 @@ __global__ __launch_bounds__(64 * NW, D == 32 && CAUSAL && NQ == 2 ? 5 : 1) void
       for (int k = 0; k < 4; ++k) op[k] = res[k];
     }
     if (a.lse && d == 0)
-      a.lse[((int64_t)b * a.Hq + h) * a.Sq + row] =
-          ltot > 0.0f ? (M + log2f(ltot)) * kLn2 : -INFINITY;
+      a.lse[((int64_t)b * a.Hq + h) * a.Sq + row] = ltot > 0.0f ? row_lse(M, ltot) : -INFINITY;
   }
 }
 

@@ -177,7 +177,7 @@ __device__ inline void store_state(const DecArgs &a, int64_t bh, int split, int 
   if (a.splits == 1) {
     // an empty sequence (paged decode with length 0) has L = 0: O = 0, lse = -inf
     a.o[bh * DH + d] = Bf16Tag::from_f32(Ls > 0.0f ? acc / Ls : 0.0f);
-    if (d == 0 && a.lse) a.lse[bh] = Ls > 0.0f ? (M + log2f(Ls)) * kLn2 : -INFINITY;
+    if (d == 0 && a.lse) a.lse[bh] = Ls > 0.0f ? row_lse(M, Ls) : -INFINITY;
     return;
   }
   const int64_t row = bh * a.splits + split;
@@ -847,7 +847,7 @@ __global__ __launch_bounds__(DH * SG) void decode_combine(const float *part_o,
   const float Ls = stat[1];
   // an empty sequence (paged decode with length 0) has L = 0: O = 0, lse = -inf
   o[bh * DH + d] = Bf16Tag::from_f32(Ls > 0.0f ? acc / Ls : 0.0f);
-  if (d == 0 && lse) lse[bh] = Ls > 0.0f ? (stat[0] + log2f(Ls)) * kLn2 : -INFINITY;
+  if (d == 0 && lse) lse[bh] = Ls > 0.0f ? row_lse(stat[0], Ls) : -INFINITY;
 }
 
 // One work-group per (batch, kv head, scale block): amax, scale, codes.

@@ -79,3 +79,19 @@ def test_fp32_sums_stay_short(B, H, D):
     chain = 2.0 ** -23 / math.sqrt(12) * 0.74 * math.sqrt(128 / 2)
     print(f"  error against 64 bits {err}, sums of 128 terms {chain:.2e}", flush=True)
     assert err[2048] <= 1.1 * math.hypot(err[128], chain)
+
+
+def test_fp32_lse_rounds_three_times():
+    """fp32 log-sum-exps of 2048 keys, around 8: an rms error of the spacing of
+    floats over sqrt(12) for the result (2^-20 from 8 on) and for the one term of
+    4 to 8 in it (2^-21), 3.1e-7 together, and 15% more for the sums."""
+    from neptune_hip import ops
+    print("case: fp32 lse", flush=True)
+    q, k, v = (randn((2, 4, 2048, 64), seed=s, dtype=torch.float32).cuda() for s in (7, 8, 9))
+    _, lse = ops.attention(q, k, v, return_lse=True)
+    ref = torch.stack([torch.logsumexp(
+        torch.matmul(q[b, h].double(), k[b, h].double().t().contiguous()) / 8.0, -1)
+        for b in range(2) for h in range(4)]).view(2, 4, 2048)
+    rms = float((lse.double() - ref).pow(2).mean().sqrt())
+    print(f"  rms error {rms:.3e}", flush=True)
+    assert rms <= 1.15 * math.hypot(2.0 ** -20, 2.0 ** -21) / math.sqrt(12)
