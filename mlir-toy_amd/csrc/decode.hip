@@ -49,9 +49,12 @@ constexpr float kSlack = 8.0f;
 // p, and the step max is not needed. Otherwise (a p above 2^kSlack, an
 // overflow, a NaN, or only a large sum) the max is formed, m moves if it
 // must, and p is taken again. The first step always forms it (m starts at
-// -FLT_MAX). A row's four lanes (lane ^ 16, ^ 32) decide together.
-__device__ inline void softmax_step(const f32x4 (&s)[2], bool first, float &m, float &lsum,
-                                    f32x4 (&oacc)[8], float (&p)[8], float &rs) {
+// -FLT_MAX). A row's four lanes (lane ^ 16, ^ 32) decide together. lift() (0
+// to 1) is how far above the step max m is put, so that the largest p takes no
+// rounding to 16 bits: 0 where p itself is rounded.
+template <class Lift>
+__device__ inline void softmax_step(const f32x4 (&s)[2], bool first, Lift lift, float &m,
+                                    float &lsum, f32x4 (&oacc)[8], float (&p)[8], float &rs) {
   auto expo = [&]() {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -72,7 +75,7 @@ __device__ inline void softmax_step(const f32x4 (&s)[2], bool first, float &m, f
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kb][r]);
     mx = max_xor32(max_xor16(mx));
     if (__any(mx > m + kSlack)) {
-      const float m_new = fmaxf(m, mx);
+      const float m_new = fmaxf(m, mx + lift());
       const float alpha = fast_exp2(m - m_new);
       m = m_new;
       lsum *= alpha;
@@ -380,7 +383,7 @@ __global__ __launch_bounds__(64 * RW) void decode_partial_ring(DecArgs a) {
           if (t + 16 * kb + 4 * G + r >= t1) s[kb][r] = -INFINITY;
     }
     float rs, p[8];
-    softmax_step(s, i == 0, m, lsum, oacc, p, rs);
+    softmax_step(s, i == 0, [] { return 0.0f; }, m, lsum, oacc, p, rs);
     lsum += rs;
     // P^T: k-slot 8 G + j holds key 4 G + j (j < 4) or 16 + 4 G + j - 4
     u32x4 pf;
@@ -716,7 +719,13 @@ __global__ __launch_bounds__(64 * R8W) void decode_partial_ring8(DecArgs a) {
           if (t + 16 * kb + 4 * G + r >= t1) s[kb][r] = -INFINITY;
     }
     float rs, p[8];
-    softmax_step(s, i == 0, m, lsum, oacc, p, rs);
+    // p vsc is rounded: its largest value is put at a power of two, where all
+    // of a wave's m would otherwise leave it at vsc's own mantissa
+    auto lift = [&] {
+      const uint32_t mant = __builtin_bit_cast(uint32_t, vsc) & 0x7fffffu;
+      return __builtin_amdgcn_logf(__builtin_bit_cast(float, mant | 0x3f800000u));
+    };
+    softmax_step(s, i == 0, lift, m, lsum, oacc, p, rs);
     lsum += rs;
     u32x4 pf;
 #pragma unroll
