@@ -375,7 +375,9 @@ __global__ __launch_bounds__(NT * KW, 2 / KW) void attn_fwd_tile(AttnArgs a, Spl
 
 // Combine of the splits' states: HD / 4 lanes per row, four head_dim elements
 // each. M = max m_s, l = sum 2^(m_s - M) l_s, O = sum 2^(m_s - M) O_s / l; a
-// split with l_s = 0 (no visible key) has left no O_s. NS (a power of two) is
+// split with l_s = 0 (no visible key) may have left no O_s and is passed over
+// (weight -1); one whose weight is 0 by underflow is not, so that an infinity or
+// NaN in its O_s reaches O as it does in an uncut launch. NS (a power of two) is
 // at least the number of splits: every O_s is loaded before the first weight
 // is known, so the row waits on memory once.
 template <class E, int HD, int NS>
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(NT) void attn_combine(AttnArgs a, SplitArgs x, int6
   float l = 0.0f;
 #pragma unroll
   for (int i = 0; i < SPL; ++i) {
-    st[i][0] = st[i][1] == 0.0f ? 0.0f : fast_exp2(st[i][0] - M);  // the split's weight
+    st[i][0] = st[i][1] == 0.0f ? -1.0f : fast_exp2(st[i][0] - M);  // the split's weight
     l = fmaf(st[i][0], st[i][1], l);
   }
 #pragma unroll
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(NT) void attn_combine(AttnArgs a, SplitArgs x, int6
   for (int s = 0; s < NS; ++s) {
     const float wgt = __shfl(st[s / LPR][0], s % LPR, LPR);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) acc[k] = wgt == 0.0f ? acc[k] : fmaf(wgt, os[s][k], acc[k]);
+    for (int k = 0; k < 4; ++k) acc[k] = wgt < 0.0f ? acc[k] : fmaf(wgt, os[s][k], acc[k]);
   }
   if (grow0 >= nrows) return;
   const int64_t bh = grow / a.Sq;

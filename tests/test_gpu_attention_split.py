@@ -73,6 +73,33 @@ def test_short_launches(B, Hq, Hk, Sq, Sk, D, causal, dtype, ws):
     assert np.abs(lse[fin] - rl[fin]).max() <= TOL_LSE_ABS
 
 
+@pytest.mark.parametrize("ws", [True, False], ids=["workspace", "none"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_non_finite_values_far_below_the_max(bad, D, ws):
+    """A V row that is not finite, at a key whose probability underflows next to
+    a later split's: the column is not finite, cut or not."""
+    from neptune_hip import ops
+    print(f"case: split V={bad} D={D} ws={ws}", flush=True)
+    q = torch.ones((1, 1, 3, D), dtype=torch.bfloat16, device="cuda")
+    k = torch.zeros((1, 1, 4000, D), dtype=torch.bfloat16, device="cuda")
+    k[:, :, 3000] = 400.0 / D ** 0.5  # 577 (log2 units) above the other keys
+    v = torch.ones_like(k)
+    v[:, :, 10, 5] = bad
+    if ws:
+        o = ops.attention(q, k, v)
+    else:
+        lib = _abi.load_library()
+        o, d = torch.empty_like(q), _desc(1, 1, 1, 3, 4000, D, False, torch.bfloat16)
+        _abi.check(lib.neptune_attn_fwd(ctypes.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                        o.data_ptr(), None,
+                                        torch.cuda.current_stream().cuda_stream), lib)
+    finite = torch.isfinite(o.cpu())
+    assert not finite[..., 5].any()
+    finite[..., 5] = True
+    assert finite.all()
+
+
 def test_workspace_too_small():
     lib = _abi.load_library()
     d = _desc(1, 4, 1, 250, 2100, 128, True, torch.bfloat16)
