@@ -490,6 +490,17 @@ __global__ __launch_bounds__(NT, 5) void selective_scan_out(ScanArgs a) {
   store_outputs(tb + (te - tb - 1) / TT * TT);  // the last chunk's
 }
 
+// The state x of one chunk's start at the end of it: 2^e x + c, c the chunk's
+// end state from 0. Its steps, one after another, leave a 0 or an infinity as it
+// is and reach a finite state where 2^e alone is past fp32 (decays above 1: A
+// or delta of the other sign), so the same holds here.
+__device__ inline float advance(float e, float x, float c) {
+  if (x == 0.0f || __builtin_isinf(x)) return x + c;
+  const bool far = e > 126.0f;
+  const float f = fast_exp2(far ? 0.5f * e : e);
+  return fmaf(f, far ? f * x : x, c);
+}
+
 // The carry pass: one lane per (batch row, channel, state) walks the chunks
 // in order and leaves each chunk's starting state where its end state was.
 // The walk depends on memory only through the chunk summaries, which do not
@@ -525,7 +536,7 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
     for (int i = 0; i < KB; ++i)
       if (k0 + i < nsum) {
         chunk_scratch(a, row_s, k0 + i)[n] = carry;
-        carry = fmaf(fast_exp2(A2 * S[set][i]), carry, xe[set][i]);
+        carry = advance(A2 * S[set][i], carry, xe[set][i]);
       }
   };
   using S0 = std::integral_constant<int, 0>;
@@ -542,8 +553,8 @@ __global__ __launch_bounds__(256) void selective_scan_carry(ScanArgs a, int32_t 
 
 // The carry pass for long chains of chunks (more than 64 summaries): one
 // wave per (batch row, channel, state), 64 chunks per pass, one per lane.
-// Chunk k maps its starting state x to a_k x + b_k (a_k = 2^(A S_k log2 e),
-// b_k its end state from 0); an inclusive scan of these affine maps across
+// Chunk k maps its starting state x to 2^e_k x + b_k (e_k = A S_k log2 e, b_k
+// its end state from 0; advance() applies it); an inclusive scan of these affine maps across
 // the lanes (Hillis-Steele, six shuffles) gives every lane the map from the
 // pass's starting state to the end of its chunk, so its chunk's starting
 // state is the previous lane's map applied to that state. The pass's loads
@@ -563,22 +574,22 @@ __global__ __launch_bounds__(256) void selective_scan_carry_wave(ScanArgs a, int
     const int k = k0 + lane;
     const bool live = k < nsum;
     const float *p = chunk_scratch(a, row_s, live ? k : nsum - 1);
-    float m = live ? fast_exp2(A2 * p[ST]) : 1.0f;  // this lane's map: x -> m x + c
+    float e = live ? A2 * p[ST] : 0.0f;  // this lane's map: x -> 2^e x + c
     float c = live ? p[n] : 0.0f;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-      // compose with the map of the lanes before: x -> m (m' x + c') + c
-      const float mp = __shfl_up(m, off, 64), cp = __shfl_up(c, off, 64);
+      // compose with the map of the lanes before: x -> 2^e (2^e' x + c') + c
+      const float ep = __shfl_up(e, off, 64), cp = __shfl_up(c, off, 64);
       if (lane >= off) {
-        c = fmaf(m, cp, c);
-        m *= mp;
+        c = advance(e, cp, c);
+        e += ep;
       }
     }
     // this chunk starts where the lanes before it end
-    const float mp = __shfl_up(m, 1, 64), cp = __shfl_up(c, 1, 64);
-    const float start = lane == 0 ? carry : fmaf(mp, carry, cp);
+    const float ep = __shfl_up(e, 1, 64), cp = __shfl_up(c, 1, 64);
+    const float start = lane == 0 ? carry : advance(ep, carry, cp);
     if (live) chunk_scratch(a, row_s, k)[n] = start;
-    carry = fmaf(__shfl(m, 63, 64), carry, __shfl(c, 63, 64));
+    carry = advance(__shfl(e, 63, 64), carry, __shfl(c, 63, 64));
   }
   if (lane == 0) chunk_scratch(a, row_s, nsum)[n] = carry;  // the last chunk's starting state
 }

@@ -60,3 +60,28 @@ def test_chunked_unaligned_rows(b, d, L, gate, softplus, shift):
     got = to_f32(y).astype(np.float64)
     assert np.isfinite(got).all()
     assert (np.abs(got - ref) <= 2e-2 * np.maximum(1.0, np.abs(ref))).all()
+
+
+@pytest.mark.parametrize("d,L", [(64, 2047), (16, 16383)], ids=["walk", "wave"])
+@pytest.mark.parametrize("sign_a,delta", [(1.0, 1.0), (-1.0, -1.0)])
+def test_growing_states(d, L, sign_a, delta):
+    """Decays above 1, whose product over a chunk (e^96 and more) fp32 does not
+    hold: states stay 0 while u is 0 and grow from where it starts, as they do
+    step by step; an infinite one stays infinite."""
+    print(f"case: scan growing d={d} L={L} A={sign_a} delta={delta}", flush=True)
+    u = randn((1, d, L), seed=1)
+    u[:, :, :L - 40] = 0
+    u[:, 0, 10] = float("inf")
+    dr = torch.full((1, d, L), delta, dtype=torch.bfloat16)
+    A = torch.full((d, 16), sign_a)
+    ones = torch.ones((1, 16, L), dtype=torch.bfloat16)
+    y = ops.selective_scan(u.cuda(), dr.cuda(), A.cuda(), ones.cuda(), ones.cuda(),
+                           delta_softplus=False)
+    ref_bits, _ = oracle.selective_scan(bits(u), bits(dr), A.numpy(), bits(ones), bits(ones),
+                                        softplus=False)
+    ref = oracle.decode(ref_bits, oracle.BF16).astype(np.float64)
+    got = to_f32(y).astype(np.float64)
+    assert not np.isfinite(got[0, 0, 10:]).any()
+    got, ref = got[0, 1:], ref[0, 1:]
+    assert np.isfinite(got).all()
+    assert (np.abs(got - ref) <= 2e-2 * np.maximum(1.0, np.abs(ref))).all()
