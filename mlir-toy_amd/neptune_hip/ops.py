@@ -28,7 +28,8 @@ _TORCH_TO_DTYPE = {
 # The checks of a call and its descriptor depend on the tensors' shapes,
 # strides, dtypes and devices and on the options alone, so each entry point
 # keeps them by those values (bounded; a call that fails its checks is not
-# kept). Working them out took 3-8 us of every call, as long as the smallest
+# kept) and by the options' types: 4.0 is no split count, equal to 4 or not.
+# Working them out took 3-8 us of every call, as long as the smallest
 # kernels run: now a lookup.
 _PLANS = 1024
 
@@ -107,7 +108,7 @@ def scale_to_log2(scale: float | None, head_dim: int) -> float:
     return float(scale) * LOG2E
 
 
-@functools.lru_cache(maxsize=_PLANS)
+@functools.lru_cache(maxsize=_PLANS, typed=True)
 def _attn_plan(q, k, v, out, lse, causal, scale, scale_log2, stages, k_dim_order):
     """(descriptor, bytes of the split states' workspace, LSE shape)."""
     _require_cuda(q, k, v, out, lse)
@@ -227,7 +228,7 @@ def _as_q3(q: torch.Tensor) -> torch.Tensor:
     return q
 
 
-@functools.lru_cache(maxsize=_PLANS)
+@functools.lru_cache(maxsize=_PLANS, typed=True)
 def _decode_plan(q, k, v, k_scale, v_scale, num_splits, scale_block, scale):
     """(descriptor, workspace bytes)."""
     fp8 = k[2] in (torch.uint8, torch.float8_e4m3fn)
@@ -299,7 +300,7 @@ def decode_splitk(
     return (out, lse) if return_lse else out
 
 
-@functools.lru_cache(maxsize=_PLANS)
+@functools.lru_cache(maxsize=_PLANS, typed=True)
 def _paged_plan(q, k_pages, v_pages, block_table, seq_lens, k_scales, v_scales, max_seq_len,
                 num_splits, scale):
     """(descriptor, page descriptor, workspace bytes, whether the pools are E4M3)."""
@@ -404,7 +405,7 @@ def kv_quantize_fp8(kv: torch.Tensor, *, scale_block: int = 64):
     return codes, scales
 
 
-@functools.lru_cache(maxsize=_PLANS)
+@functools.lru_cache(maxsize=_PLANS, typed=True)
 def _scan_plan(u, delta, A, B, C, D, z, delta_bias, delta_softplus):
     """The descriptor."""
     for name, m in (("u", u), ("delta", delta), ("B", B), ("C", C), ("z", z)):

@@ -7,6 +7,7 @@ drive them with meta tensors (no storage, no GPU) and expect ValueError,
 the class the reference raises for bad input.
 """
 
+import numpy as np
 import pytest
 import torch
 
@@ -142,3 +143,21 @@ def test_scan_shape_checks(name, shape, dtype):
     args[name] = meta(shape, dtype)
     with pytest.raises(ValueError, match=name):
         ops.selective_scan(**args)
+
+
+@pytest.mark.parametrize("bad", [4.0, np.int64(4)])
+def test_kept_plan_does_not_admit_equal_options_of_other_types(bad):
+    """A split count that is no int is refused, also after a call with the equal
+    int has left its plan (plans need no GPU: a device by name only)."""
+    dev = torch.device("cuda", 0)
+    q = (torch.Size((2, 8, 128)), (1024, 128, 1), bf16, dev)
+    kv = (torch.Size((2, 2, 256, 128)), (65536, 32768, 128, 1), bf16, dev)
+    ops._decode_plan(q, kv, kv, None, None, 4, 64, None)
+    with pytest.raises(TypeError):
+        ops._decode_plan(q, kv, kv, None, None, bad, 64, None)
+    table = (torch.Size((2, 4)), (4, 1), i32, dev)
+    lens = (torch.Size((2,)), (1,), i32, dev)
+    pages = (torch.Size((8, 2, 64, 128)), (16384, 8192, 128, 1), bf16, dev)
+    ops._paged_plan(q, pages, pages, table, lens, None, None, 256, 4, None)
+    with pytest.raises(TypeError):
+        ops._paged_plan(q, pages, pages, table, lens, None, None, 256, bad, None)
