@@ -7,7 +7,6 @@ drive them with meta tensors (no storage, no GPU) and expect ValueError,
 the class the reference raises for bad input.
 """
 
-import numpy as np
 import pytest
 import torch
 
@@ -145,8 +144,7 @@ def test_scan_shape_checks(name, shape, dtype):
         ops.selective_scan(**args)
 
 
-@pytest.mark.parametrize("bad", [4.0, np.int64(4)])
-def test_kept_plan_does_not_admit_equal_options_of_other_types(bad):
+def test_kept_plan_does_not_admit_an_equal_float():
     """A split count that is no int is refused, also after a call with the equal
     int has left its plan (plans need no GPU: a device by name only)."""
     dev = torch.device("cuda", 0)
@@ -154,10 +152,10 @@ def test_kept_plan_does_not_admit_equal_options_of_other_types(bad):
     kv = (torch.Size((2, 2, 256, 128)), (65536, 32768, 128, 1), bf16, dev)
     ops._decode_plan(q, kv, kv, None, None, 4, 64, None)
     with pytest.raises(TypeError):
-        ops._decode_plan(q, kv, kv, None, None, bad, 64, None)
+        ops._decode_plan(q, kv, kv, None, None, 4.0, 64, None)
     table = (torch.Size((2, 4)), (4, 1), i32, dev)
     lens = (torch.Size((2,)), (1,), i32, dev)
     pages = (torch.Size((8, 2, 64, 128)), (16384, 8192, 128, 1), bf16, dev)
     ops._paged_plan(q, pages, pages, table, lens, None, None, 256, 4, None)
     with pytest.raises(TypeError):
-        ops._paged_plan(q, pages, pages, table, lens, None, None, 256, bad, None)
+        ops._paged_plan(q, pages, pages, table, lens, None, None, 256, 4.0, None)
