@@ -59,8 +59,8 @@ def test_config1_fp32_matches_oracle(ops):
     (1, 1, 1, 200, 150, 64, True),    # more queries than keys: early rows see no key
 ])
 def test_fp32_shapes_match_oracle(ops, B, Hq, Hk, Sq, Sk, D, causal):
-    """The fp32 path (16 lanes per query row, each over every 16th key, merged
-    at the end) at 1e-5 relative of the oracle, LSE included; rows with no
+    """The fp32 path (the keys shared out between the waves of a block of query
+    rows, merged at the end) at 1e-5 relative of the oracle, LSE included; rows with no
     visible key give O = 0 and LSE = -inf."""
     _log(f"case: fp32 B={B} Hq={Hq} Hk={Hk} Sq={Sq} Sk={Sk} D={D} causal={causal}")
     q = randn((B, Hq, Sq, D), seed=11, dtype=torch.float32)

@@ -21,7 +21,9 @@ SHAPES = [  # B, Hq, Hk, Sq, Sk, D, causal
     (1, 8, 2, 3, 1500, 128, True),     # packed rows of three positions, one row block
     (2, 8, 1, 40, 700, 128, True),     # packed: heads change inside a wave's rows
     (1, 2, 2, 900, 900, 128, True),    # early row blocks leave later splits empty
-    (1, 2, 1, 700, 300, 128, True),    # rows that see no key
+    (1, 2, 1, 700, 300, 128, True),    # too few key blocks: not cut; rows that see no key
+    (1, 2, 2, 900, 700, 128, True),    # cut, with rows that see no key of any split
+    (1, 2, 2, 700, 600, 64, True),
     (1, 2, 2, 130, 1000, 128, False),  # no mask, one row past a block
     (1, 2, 2, 300, 130, 128, False),   # no mask, one split, single blocks
     (3, 6, 2, 1, 64 * 9 + 1, 64, False),
@@ -58,6 +60,7 @@ def test_short_launches(B, Hq, Hk, Sq, Sk, D, causal, dtype, ws):
     if ws:
         n = ctypes.c_size_t()
         _abi.check(lib.neptune_attn_workspace_bytes(ctypes.byref(d), ctypes.byref(n)), lib)
+        assert (n.value > 0) == (Sk > 300)  # cut, from ten key blocks on here
         buf = torch.full((n.value // 4 + 4,), float("nan"), device="cuda")
         _abi.check(lib.neptune_attn_fwd_ws(*args, buf.data_ptr(), n.value, stream), lib)
     else:

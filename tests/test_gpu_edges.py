@@ -3,9 +3,10 @@
 - Decode with caches shorter than one 32-token step, one token past a step,
   and more splits than steps: the layout then leaves whole splits empty,
   and the combine must weigh them zero.
-- The head_dim-128 prefill kernel with one query row, one key, and more
-  queries than keys under the causal mask. The early rows then see no key
-  at all and must give O = 0 and LSE = -inf.
+- Short head_dim-128 prefill with one query row (packed, and cut along the
+  keys where they are many), one key, and more queries than keys under the
+  causal mask. The early rows then see no key at all and must give O = 0 and
+  LSE = -inf.
 - The selective scan at sequence lengths 1, 2 and 3 and one step either side
   of its 32-step chunk, over a channel count that leaves a partial channel
   block.

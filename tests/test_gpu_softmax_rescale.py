@@ -11,10 +11,16 @@ built so that, against q of all ones, the log2-domain scores step through:
   block 12      +248 on every other key: p = 2^6 each, so a lane's sum
                 passes 2^8 while no p does (the max is formed, m stays)
   blocks 13-    +239
-Prefill (head_dim 128, bf16 and f16, causal and not) and split-K decode
-(bf16 and fp8 KV, splits that start inside the ramp) are checked against the
-CPU oracle, which takes the plain running max.
+Prefill (bf16, f16 and fp32) and split-K decode (bf16 and fp8 KV, splits that
+start inside the ramp) are checked against the CPU oracle, which takes the plain
+running max. The prefill launches are such that one chain of key blocks holds
+the whole ramp: a launch that fills the GPU, one cut into splits of 16 key
+blocks or more, and one whose halves of the keys go to four waves each (32 key
+blocks, without a workspace); 1024 keys of two heads are cut into splits of two
+key blocks, each of which starts inside the ramp.
 """
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -22,6 +28,8 @@ import torch
 
 import oracle
 from helpers import TOL_BF16_ABS, TOL_FP8_ABS, TOL_LSE_ABS, bits, max_abs, oracle_dtype, to_f32
+from neptune_hip import _abi
+from test_gpu_attention_large import check_heads
 
 pytestmark = pytest.mark.gpu
 
@@ -53,11 +61,11 @@ def ramp_targets(L):
     return t
 
 
-def ramp_kv(B, H, L, seed, dtype):
+def ramp_kv(B, H, L, seed, dtype, dim=D):
     g = torch.Generator().manual_seed(seed)
-    base = (ramp_targets(L) / LOG2_PER_UNIT).view(1, 1, L, 1)
-    k = base + 0.05 * torch.randn((B, H, L, D), generator=g)
-    v = torch.randn((B, H, L, D), generator=g)
+    base = (ramp_targets(L) / (LOG2_PER_UNIT * (dim / D) ** 0.5)).view(1, 1, L, 1)
+    k = base + 0.05 * torch.randn((B, H, L, dim), generator=g)
+    v = torch.randn((B, H, L, dim), generator=g)
     return k.to(dtype), v.to(dtype)
 
 
@@ -81,6 +89,63 @@ def test_prefill_climbing_scores(ops, causal, dtype):
     assert np.isfinite(got).all()
     assert max_abs(got, ref) <= TOL_BF16_ABS * max(1.0, np.abs(ref).max())
     assert max_abs(to_f32(lse), rl) <= TOL_LSE_ABS
+
+
+@pytest.mark.parametrize("form,B,Hq,Hk,Sq,Sk,dim", [
+    ("whole", 4, 32, 32, 1024, 1024, 128),
+    ("whole", 8, 16, 16, 1024, 1024, 64),
+    ("splits", 1, 32, 8, 250, 8000, 128),
+    ("splits", 2, 32, 8, 250, 8000, 64),
+    ("halves", 1, 2, 2, 2048, 2048, 128),
+    ("halves", 1, 2, 2, 2048, 2048, 64),
+])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prefill_forms_climbing_scores(ops, form, B, Hq, Hk, Sq, Sk, dim, causal, dtype):
+    _log(f"case: prefill {form} climbing scores B={B} {Hq}/{Hk} {Sq}x{Sk} D={dim} "
+         f"causal={causal} dtype={dtype}")
+    q = ramp_q((B, Hq, Sq, dim), 7, dtype).cuda()
+    k, v = (t.cuda() for t in ramp_kv(B, Hk, Sk, 8, dtype, dim))
+    lib = _abi.load_library()
+    d, n = _abi.AttnDesc(), ctypes.c_size_t()
+    d.batch, d.heads_q, d.heads_kv, d.seq_q, d.seq_kv, d.head_dim = B, Hq, Hk, Sq, Sk, dim
+    d.dtype = _abi.DTYPE_BF16 if dtype == torch.bfloat16 else _abi.DTYPE_F16
+    d.causal = int(causal)
+    _abi.check(lib.neptune_attn_workspace_bytes(ctypes.byref(d), ctypes.byref(n)), lib)
+    if form == "splits":  # at most Sk / 1024 of them, so 16 key blocks or more in each
+        assert 0 < n.value <= B * Hq * Sq * (Sk // 1024 + 1) * (dim + 2) * 4
+    elif form == "whole":
+        assert n.value == 0
+    if form == "halves":
+        o = torch.empty_like(q)
+        lse = torch.empty((B, Hq, Sq), device="cuda")
+        _abi.check(lib.neptune_attn_fwd(ctypes.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                        o.data_ptr(), lse.data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream), lib)
+    else:
+        o, lse = ops.attention(q, k, v, causal=causal, return_lse=True)
+    check_heads(q, k, v, o, lse, causal)
+
+
+@pytest.mark.parametrize("B,H,S", [(4, 32, 1024), (1, 2, 2048)], ids=["four_waves", "eight_waves"])
+@pytest.mark.parametrize("dim", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fp32_climbing_scores(ops, B, H, S, dim, causal):
+    """Scores of 248 (log2 units) come from sums of up to 128 products, each
+    rounded, in the kernel and in the oracle: 2^-24 sqrt(128) of them, which p
+    takes times ln 2: 1.2e-4 each."""
+    _log(f"case: fp32 climbing scores B={B} H={H} S={S} D={dim} causal={causal}")
+    q = ramp_q((B, H, S, dim), 9, torch.float32).cuda()
+    k, v = (t.cuda() for t in ramp_kv(B, H, S, 10, torch.float32, dim))
+    o, lse = ops.attention(q, k, v, causal=causal, return_lse=True)
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        qq, kk, vv = (t[b, h][None, None].cpu() for t in (q, k, v))
+        ro, rl = oracle.attn_fwd(bits(qq), bits(kk), bits(vv), oracle.F32, causal)
+        ref = oracle.decode(ro, oracle.F32)[0, 0]
+        got = to_f32(o[b, h])
+        assert np.isfinite(got).all()
+        assert max_abs(got, ref) <= 2.4e-4 * np.abs(ref).max()
+        assert max_abs(to_f32(lse[b, h]), rl[0, 0]) <= TOL_LSE_ABS
 
 
 @pytest.mark.parametrize("splits", [1, 3])

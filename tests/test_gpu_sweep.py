@@ -15,9 +15,9 @@ checks the result against the CPU oracle at the contract's tolerances:
   32-256, both pool layouts, bf16 and fp8 pools, ragged lengths including
   empty sequences;
 * selective scan (neptune_selective_scan_fwd): batch 1-3, ragged channel
-  counts, lengths 1-1500 (odd ones take the single pass, even ones of two
-  64-step chunks or more the chunked path when the channels leave the GPU
-  unfilled), with or without z, D and delta_bias, softplus on or off; and
+  counts, lengths 1-1500 (those of four 32-step units or more, odd or even,
+  take the chunked path where the channels leave the GPU unfilled and its
+  estimate is the lower), with or without z, D and delta_bias, softplus on or off; and
   eight long few-channel cases (lengths 2048-24000, 1-47 channels), whose
   chains of more than 64 chunks take the wave-parallel carry.
 """

@@ -320,6 +320,15 @@ BUDGETS = [
     (r"selective_scan_out", 96, "five waves per SIMD"),
     # the production prefill (two LDS stages): two work-groups per CU
     (r"attn_fwd_d128INS_7Bf16TagELb1ELi2ELb0E", 256, "two waves per SIMD"),
+    # head_dim 64 and the cut launches: two four-wave work-groups per CU (one of
+    # eight waves)
+    (r"attn_fwd_tile", 256, "two waves per SIMD"),
+    # fp32 with 32-row work-groups: what each fits beside its LDS
+    (r"attn_fwd_f32ILi32ELb[01]ELi2E", 96, "five waves per SIMD"),
+    (r"attn_fwd_f32ILi64ELb[01]ELi2E", 168, "three waves per SIMD"),
+    (r"attn_fwd_f32ILi128ELb[01]ELi2E", 256, "two waves per SIMD"),
+    # and with 16-row ones of eight waves
+    (r"attn_fwd_f32ILi\d+ELb[01]ELi1E", 168, "three waves per SIMD"),
     # the decode partial kernels: a scratch reload's wait would retire the
     # copies in flight
     (r"decode_partial_ring", 512, "no scratch"),
