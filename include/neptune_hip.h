@@ -77,9 +77,13 @@ typedef struct neptune_backend_info {
  * reads (lib/HTile/HTilePasses.cpp:122-140). pipeline_stages is the number
  * of K and V tiles the kernel keeps in LDS per operand, i.e. how far its
  * loads run ahead (the htile.pipeline_stages loop attribute, HTile:128);
- * neither knob changes the result. Both apply to the head_dim-128 16-bit
- * kernel (0 = default elsewhere; launches too short to fill the GPU always
- * keep two tiles); k_dim_order = 1 needs seq_kv % 8 == 0. Query head h reads KV head h / (heads_q / heads_kv).
+ * it does not change the result. Both knobs apply to the head_dim-128 16-bit
+ * kernel (0 = default elsewhere; launches of at most 512 blocks of 128 query
+ * rows, too short to fill the GPU, may run a kernel that keeps two tiles,
+ * whatever the stage count, unless k_dim_order is 1). k_dim_order = 1 needs seq_kv % 8
+ * == 0; such launches are never cut (below), so against order 0 their results
+ * may differ as the two forms of a cut launch do. Query head h reads KV head
+ * h / (heads_q / heads_kv).
  * Numerics follow tests/data/flash_attention_htile.mlir:23-143: scores are
  * scaled by scale_log2 (= log2(e)/sqrt(D) when 0, HTile:24) into the exp2
  * domain, the running max starts at -FLT_MAX, keys stream in blocks of 64,
@@ -178,8 +182,11 @@ NEPTUNE_API neptune_status neptune_attn_fwd(const neptune_attn_desc *desc, const
  * launch is not split and workspace may be NULL); a smaller or missing
  * workspace is NEPTUNE_ERR_WORKSPACE_TOO_SMALL. The workspace needs no
  * clearing, must be 16-byte aligned and is in use until the call's work on
- * `stream` is done. Arguments, results and errors are otherwise
- * neptune_attn_fwd's; results differ from it by fp32 rounding of the sums. */
+ * `stream` is done. Arguments and errors are otherwise neptune_attn_fwd's.
+ * Results differ from it by rounding: each split has a running max of its own,
+ * against which its probabilities are rounded to the input type, so outputs
+ * may differ by that rounding (about 3e-3 relative in bf16, 4e-4 in f16); both
+ * forms are as close to the exact result. */
 NEPTUNE_API neptune_status neptune_attn_workspace_bytes(const neptune_attn_desc *desc,
                                             size_t *bytes);
 

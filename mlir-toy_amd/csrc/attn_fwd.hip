@@ -63,10 +63,12 @@ constexpr int F32_STRETCH = 6;
 // the line the GPU is short of work-groups and a wave's serial key loop sets
 // the time, so 16-row work-groups cut the keys eight ways; above it the
 // matrix units are full and 32-row work-groups of 4 waves read K and V half
-// as often. Measured at D = 64 (us, 16-row / 32-row): no mask 128 blocks
-// 15.4 / 22.8, 256 blocks 28.3 / 24.8; causal, where the late blocks hold
-// most of the work, 256 blocks 21.1 / 22.9, 512 blocks 21.5 / 19.6 (S 512)
-// and 32.1 / 33.3 (S 1024). D = 32 and 128 cross at the same counts.
+// as often. Measured (us, 16-row / 32-row; D = 64, then 32 and 128): no mask 128
+// blocks (8 heads, S 512) 9.8 / 14.0, 6.5 / 8.8, 16.6 / 23.6; 256 (16 heads)
+// 16.6 / 14.9, 10.2 / 9.5, 30.6 / 24.3; causal, where the late blocks hold most of
+// the work, 256 13.5 / 14.5, 8.5 / 9.1, 23.0 / 24.2; 512 (32 heads) 22.4 / 19.2,
+// 13.7 / 11.9, 42.9 / 33.5; 512 (16 heads, S 1024) 32.3 / 31.0, 20.5 / 18.8, 62.4
+// / 56.0.
 constexpr int64_t F32_FILL = 256, F32_FILL_CAUSAL = 512;
 
 template <int N>
@@ -134,9 +136,9 @@ __global__ __launch_bounds__(64 * NW, D == 32 && CAUSAL && NQ == 2 ? 5 : 1) void
   }
 
   // VEC: a block's rows are read through a buffer resource that begins with the
-  // block and ends with the tensor's last row, so a lane's offsets are fixed
-  // and rows past the end read 0. Otherwise rows past the end read the last
-  // one. Either way no load is guarded, and such keys are masked.
+  // block and ends with its last row that exists (f32_rows), so a lane's offsets
+  // are fixed and rows past the end read 0. Otherwise rows past the end read the
+  // tensor's last one. Either way no load is guarded, and such keys are masked.
   const int krow = i * (int)a.ks2 + 4 * g, vcol = VW * i, vrow = (int)a.vs2;
   f32x4 kf[NM];
   auto load_k = [&](int kb) {
@@ -231,8 +233,9 @@ __global__ __launch_bounds__(64 * NW, D == 32 && CAUSAL && NQ == 2 ? 5 : 1) void
     for (int n = 0; n < NQ; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[n][r] += s2[n][r];
-    // unconditionally (past the last block it re-reads the last key): a
-    // branch would make the compiler wait for these loads before P.V
+    // unconditionally (past the last block the rows are zeros, or the tensor's
+    // last one again): a branch would make the compiler wait for these loads
+    // before P.V
     load_k(kb + NW);
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
@@ -441,7 +444,9 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
   }
   // a dispatch covers at most 2^32 - 1 work-items: one 256-thread work-group
   // per 128 query rows and (batch, head) (the most any 16-bit path launches),
-  // one 256-thread work-group per 16 rows for fp32 (twice what it launches)
+  // one 256-thread work-group per 16 rows for fp32 (twice what the 32-row form
+  // launches; the 16-row form, 512 threads per 16 rows, is kept to fewer than
+  // F32_FILL_CAUSAL 32-row blocks, 2^19 work-items)
   const int64_t rows = a.dtype == 0 ? 16 : 128;
   if ((a.seq_q + rows - 1) / rows * (a.batch * a.heads_q) * 256 > (int64_t)0xffffffff) {
     *why = "batch*heads*seq_q too large for one launch";
@@ -459,28 +464,30 @@ bool attn_supported(const AttnLaunch &a, const char **why) {
 //   block across two heads would see the keys of the later head's last rows.
 // - Splits: a work-group's time is its chain of 64-key blocks, so with at most
 //   one work-group per CU the chain is cut. The count is the one with the
-//   least estimated time, from what the kernels measured: a key block takes
-//   1.05 us alone on a CU and 1.65 us beside another work-group (head_dim 64:
-//   0.94 and 1.35), a launch 3 us, the combine 4.5 us, and the states
-//   move at 5 TB/s. A cut has to promise 5%. Measured (us, one piece /
-//   chosen cut / its count): 1 x 32/8 heads, 250 queries over 8000 keys 134 /
-//   44.5 / 8; 500 over 4000 71 / 44 / 4; 1 x 8 heads, 128 over 12000 197 / 22
-//   / 27; 8 x 32/4 heads, 1 over 4000 68 / 17 / 16; head_dim 64, 1 x 16/4,
-//   250 over 8000 125 / 28.4 / 8; 1 x 4, 2048 over 2048 causal 35.9 / 18.7 / 4;
-//   3 x 4, 2 over 430 9.6 / 6.8 / 7. Where it stays whole: 1 x 32 heads, 1000 over
-//   1000 causal 22.8 / 30.1 with two splits; 1 x 32/8, 256 over 512 13.9 / 17.1.
+//   least estimated time: a key block takes 1.05 us alone on a CU and 1.65 us
+//   beside another work-group (head_dim 64: 0.94 and 1.35), a launch 3 us, the
+//   combine 4.5 us, and the states move at 5 TB/s. Measured alone 1.04 (0.95),
+//   beside another 1.65 to 2.0 (1.35 to 1.5) with K and V from memory. A cut has
+//   to promise 5%. Measured (us, one piece / chosen cut / its count): 1 x 32/8
+//   heads, 250 queries over 8000 keys 135 / 47.2 / 8; 500 over 4000 71 / 46 / 4;
+//   1 x 8 heads, 128 over 12000 197 / 23.3 / 27; 8 x 32/4 heads, 1 over 4000 68 /
+//   17.7 / 16; head_dim 64, 1 x 16/4, 250 over 8000 126 / 27.8 / 16; 1 x 4, 2048
+//   over 2048 causal 35.9 / 18.9 / 8; 3 x 4, 2 over 430 9.6 / 6.9 / 7. Where it
+//   stays whole: 1 x 32 heads, 1000 over 1000 causal 23.0 / 31.7 with two splits;
+//   1 x 32/8, 256 over 512 14.6 / 17.9 (head_dim 64: 18.5 / 25.5, 11.3 / 13.1).
 // - Halves: a launch of at most one work-group per CU that stays whole has
 //   eight waves per work-group, four on each half of the keys, merged in LDS.
 //   The waves of a SIMD run in step, so their matrix and vector work overlaps
-//   less than two work-groups' (1.75 us a block pair, 1.5 us for the merge;
-//   under splits it lost to more of them: 500 over 4000 56.7 / 45.5). Measured
-//   (us, four waves / eight): 1 x 16 heads causal S 1500 30.1 / 25.6, S 2000
-//   38.4 / 32.1, 1 x 32 S 1000 22.8 / 20.6, S 640 16.4 / 15.9, S 512 14.2 /
-//   14.2; head_dim 64 (1.3 us a pair) S 2000 35.5 / 28.2, 1 x 32 S 1000 20.8 /
-//   17.7, S 512 12.7 / 11.8.
+//   less than two work-groups' (1.75 us a block pair, 1.3 at head_dim 64, and
+//   1.5 us for the merge; under splits it lost to more of them: 500 over 4000
+//   58.1 / 46). Measured (us, four waves / eight): 1 x 16 heads causal S 1500
+//   31.1 / 27.3, S 2000 39.1 / 33.8, 1 x 32 S 1000 23.5 / 22.1, S 640 17.1 /
+//   16.9, S 512 14.9 / 15.3 (too few blocks: four); head_dim 64 S 1500 28.1 /
+//   22.9, S 2000 35.9 / 28.6, 1 x 32 S 1000 21.0 / 18.0, S 640 14.9 / 13.3, S 512
+//   12.7 / 11.8.
 // - Without the mask the head_dim-128 kernel runs two query blocks per
 //   work-group; up to 512 blocks they are better apart (1 x 4 heads, 512
-//   over 512: 25.0 / 13.4).
+//   over 512: 25.3 / 13.8).
 AttnSplit attn_split(const AttnLaunch &L, bool partials) {
   AttnSplit p;
   if (L.dtype == 0 || L.k_dim_order != 0) return p;

@@ -173,8 +173,8 @@ __device__ inline int seq_chunk(const DecArgs &a, int Lb) {
 // A split's state of one (batch, query head) row, element d: the partials for
 // the combine, or, with a single split, the outputs as the combine forms them
 // (weight 1): a launch of one split needs no second kernel (us with / without
-// it: bf16 B1 32/8 heads L200 6.9 / 4.3, B16 L250 8.4 / 5.6, fp8 paged B12 8/8
-// L178 7.6 / 4.8).
+// it: bf16 B1 32/8 heads L200 7.7 / 5.2, B16 L250 9.6 / 6.8, fp8 paged B12 8/8
+// L178 8.3 / 5.4).
 __device__ inline void store_state(const DecArgs &a, int64_t bh, int split, int d, float acc,
                                    float M, float Ls) {
   if (a.splits == 1) {
@@ -800,8 +800,8 @@ __global__ __launch_bounds__(64 * R8W) void decode_partial_ring8(DecArgs a) {
 // Bound: a small kernel's launch (3-5 us) and, with one group, a dependent
 // round trip for every 8 splits past the first 16: SG keeps it to the first
 // loads up to 128 splits. Measured (us, the whole decode call, one group /
-// SG): 128 splits, B1 32/8 heads L32768 bf16 28.8 / 25.6, fp8 20.6 / 17.3; 125
-// splits, B1 8/1 L32000 fp8 14.4 / 9.9; 32 splits, B4 32/8 L8192 26.2 / 25.3.
+// SG): 128 splits, B1 32/8 heads L32768 bf16 32.1 / 29.0, fp8 23.6 / 20.4; 125
+// splits, B1 8/1 L32000 fp8 15.3 / 10.5; 32 splits, B4 32/8 L8192 29.1 / 27.9.
 constexpr int kCombinePre = 16;
 
 template <int SG>
@@ -995,9 +995,9 @@ bool decode_supported(const DecodeLaunch &a, const char **why) {
 // shared by several waves (merged in LDS). Once every CU holds the four or five
 // single-wave work-groups its LDS fits, more waves only add merges. Measured
 // (us, 1 / 2 / 4 waves): bf16, 136 work-groups of 256 tokens (B1 32/8 heads
-// L4100) 10.7 / 8.5 / 7.9, 512 of them (B2 L8192) 16.0 / 15.1 / 17.4, 1024
-// (B1 L32768) 29.7 / 30.6 / 34.9; fp8, whose ring takes half the LDS, 512
-// 13.4 / 12.9 / 11.6, 1024 21.9 / 21.9 / 22.6.
+// L4100) 12.0 / 9.8 / 9.8, 512 of them (B2 L8192) 17.6 / 17.2 / 19.1, 1024
+// (B1 L32768) 28.3 / 29.0 / 33.2; fp8, whose ring takes half the LDS, 512
+// 14.7 / 14.5 / 13.5, 1024 20.2 / 20.1 / 20.5.
 int decode_waves(int64_t groups, bool fp8) {
   if (groups <= (fp8 ? 512 : 256)) return 4;
   return groups <= 512 ? 2 : 1;
@@ -1040,11 +1040,11 @@ hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
   // where a work-group is long, or where the launch takes more than one round
   // (five bf16 work-groups per CU); sorting, some 1 us of a launch's start,
   // where it is long (one lane per sequence, its length and index in 32 bits).
-  // Measured (us, before / scaled / sorted too, lengths an eighth to all of
-  // L): fp8 B32 32/8 heads L8192 77.5 / 67.9 / 62.8, B64 L4096 77.5 / - /
-  // 63.5, token-major B29 L7497 81.2 / 74.0 / 69.7, bf16 B16 L16384 114 / - /
-  // 104, B8 L8192 (256-token work-groups, 2048 of them) 34.9 / 33.0 / 35.0;
-  // without either, bf16 B4 16/4 L20000 (1264 of 256 tokens) 28.2 / 29.6.
+  // Measured (us, neither / scaled / sorted too, lengths an eighth to all of
+  // L): fp8 B32 32/8 heads L8192 78.6 / 67.9 / 63.7, B64 L4096 78.3 / 70.7 /
+  // 64.6, token-major B29 L7497 80.5 / 77.6 / 73.4, bf16 B16 L16384 120 / 116 /
+  // 109, B8 L8192 (256-token work-groups, 2048 of them) 37.9 / 35.8 / 37.3;
+  // left alone, bf16 B4 16/4 L20000 (1264 of 256 tokens) 27.9 / 27.3 / 27.0.
   a.scaled = paged && (L.chunk >= 512 || grid > 1280);
   a.sorted = paged && L.batch > 1 && L.batch <= 64 && L.chunk >= 512 && L.seq_kv < 1 << 25;
   const int rw = decode_waves(grid, L.kv_dtype == 3);

@@ -99,11 +99,6 @@ __device__ inline float row_lse(float m, float l) {
   return fmaf(m, kLn2, fmaf((float)e, kLn2, logf(f)));
 }
 
-// value of lane (l ^ 32)
-__device__ inline float swap_halves(float x) {
-  return __shfl_xor(x, 32, 64);
-}
-
 // max(x, x of lane l ^ 16) and max(x, x of lane l ^ 32), in registers: with
 // both operands x, v_permlane16_swap exchanges rows 0 <-> 1 and 2 <-> 3 (16
 // lanes each) and v_permlane32_swap the two 32-lane halves, so one of the

@@ -609,9 +609,9 @@ __global__ __launch_bounds__(256) void selective_scan_carry_wave(ScanArgs a, int
 // work-groups of the single pass gains nothing from chunks, which do 1.6
 // times the work; and chunks past 1280 work-groups (five per CU) would run a
 // second round for a few. Measured (us, single / the count chosen here): B1
-// D2048 L2047 69.3 / 41.4, B3 D444 L817 29.1 / 19.6, B6 D660 L4637 153 / 130;
-// where the single pass stays, against chunks: B2 D3511 L3465 150 / 179, B1
-// D2260 L539 20.0 / 22.6, B2 D548 L227 10.4 / 14.2.
+// D2048 L2047 69.2 / 45.0, B3 D444 L817 29.6 / 22.2, B6 D660 L4637 154 / 142;
+// where the single pass stays, against two chunks: B2 D3511 L3465 152 / 184, B1
+// D2260 L539 20.7 / 28.4, B2 D548 L227 10.7 / 15.3.
 constexpr int64_t kScanFillGroups = 1024, kScanMaxGroups = 1280, kScanMinUnits = 2;
 constexpr int64_t kScanMaxSeq = (int64_t)1 << 26;  // 16 rows x 2 bytes x 2^26 = 2^31
 

@@ -170,7 +170,10 @@ def attention(
     ``pipeline_stages`` (0 = default 2, or 1..3) sets how many K/V tiles the
     kernel stages in LDS ahead of use; with ``k_dim_order=1`` k is given as
     [B, Hkv, D, Skv] (seq contiguous), the order of a dimension_order =
-    [1, 0] tile load. Neither changes the result.
+    [1, 0] tile load. The stage count does not change the result, and short
+    launches may keep two tiles whatever it says. Short launches with
+    ``k_dim_order=0`` may be cut along the keys and those with 1 are not, so
+    their results may differ by the 16-bit rounding of the probabilities.
     """
     if scale is not None and scale_log2 is not None:
         raise ValueError("give scale or scale_log2, not both")
