@@ -109,7 +109,7 @@ def test_config4_full_shape(ops):
 
 
 # config 4 (the single pass) and a few channels over a long sequence (the
-# sequence-parallel path: 320 chunks, the wave-parallel carry)
+# sequence-parallel path: 256 chunks, the wave-parallel carry)
 FULL_SHAPES = [(4, 5120, 2048), (1, 64, 65536)]
 
 
@@ -165,20 +165,41 @@ def test_scan_full_size_skip_term_only(ops, case, shape):
     assert (err <= ulp).all(), (float(err.max()), int((err > ulp).sum()))
 
 
+def _chunks(b, d, L):
+    """How many chunks the library cuts this shape into (the rule of
+    scan_chunking in scan.hip: the count with the least estimated time, where
+    fewer than 1024 work-groups of 16 channels and at least four 32-step units
+    leave a choice)."""
+    groups, units = -(-d // 16) * b, L // 32
+    if groups >= 1024 or units < 4:
+        return 1
+
+    def cost(n):
+        state = 32 * -(-units // n)
+        out = max(state, 32 * (units // n) + L % 32)
+        t = 2500 + out * (600 + 430 * -(-groups * n // 256)) // 32
+        if n > 1:
+            t += 6500 + state * (350 + 330 * -(-groups * (n - 1) // 256)) // 32
+        return t
+
+    best, best_t = 1, cost(1) * 95 // 100
+    for n in range(2, min(1280 // groups, units // 2) + 1):
+        if cost(n) < best_t:
+            best, best_t = n, cost(n)
+    return best
+
+
 def _chunked(b, d, L):
-    """Whether the library takes the sequence-parallel path for this shape
-    (the rule of scan_chunking in scan.hip: fewer than 1024 work-groups of 16
-    channels, an even length and at least two 64-step chunks)."""
-    groups = -(-d // 16) * b
-    return L % 2 == 0 and groups < 1024 and L >= 128
+    return _chunks(b, d, L) > 1
 
 
 @pytest.mark.parametrize("b,d,L,bias,gate", [
-    (1, 64, 65536, True, True),    # 4 channel blocks over a long sequence: 320 chunks
-    (2, 20, 9000, True, True),     # 140 chunks: the wave carry's two full passes and a part
+    (1, 64, 65536, True, True),    # 4 channel blocks over a long sequence: 256 chunks
+    (2, 20, 9000, True, True),     # 94 chunks: the wave carry's full pass and a part
     (1, 16, 4096, False, True),    # one channel block, 64 chunks of 64 steps
     (2, 48, 1000, True, False),    # ragged channel block, chunks of 96, 64 and 72 steps
-    (1, 8, 130, True, True),       # two chunks, the second 66 steps
+    (1, 8, 398, True, True),       # six chunks of 64 steps, the last 14 longer
+    (3, 1792, 1430, True, True),   # three chunks: two of 480 steps, one of 470
 ])
 def test_scan_sequence_parallel_matches_oracle(ops, b, d, L, bias, gate):
     """The chunked path (state pass, carry pass, output pass, with y as the
@@ -200,10 +221,10 @@ def test_scan_sequence_parallel_matches_oracle(ops, b, d, L, bias, gate):
     assert not bad.any(), (np.argwhere(bad)[:5], np.abs(got - ref).max())
 
 
-@pytest.mark.parametrize("b,d,L", [(1, 32, 129), (4, 4096, 256), (2, 64, 126)])
+@pytest.mark.parametrize("b,d,L", [(1, 32, 129), (4, 4096, 256), (2, 64, 126), (1, 8, 130)])
 def test_scan_single_pass_matches_oracle(ops, b, d, L):
-    """Shapes the single pass keeps: an odd length, enough channel blocks to
-    fill the GPU, and a sequence too short for two chunks."""
+    """Shapes the single pass keeps: enough channel blocks to fill the GPU, a
+    sequence too short for two chunks, and ones whose chunks would not pay."""
     assert not _chunked(b, d, L)
     _log(f"case: scan single pass b={b} d={d} L={L}")
     ins = scan_inputs(b, d, L, seed=300 + L)
@@ -255,9 +276,9 @@ def test_scan_softplus_branches(ops, b, d, L, softplus):
 @pytest.mark.parametrize("L", [(1 << 26) - 2, (1 << 26) - 1])
 def test_scan_longest_sequence_closed_form(L):
     """seq_len just below the 2^26 limit, where a 16-channel block spans
-    nearly 2^31 bytes of the kernels' 32-bit offsets: the even length takes
-    the chunked path (about 1280 chunks), the odd one the single pass (one
-    work-group walking the whole sequence). The inputs have a closed form:
+    nearly 2^31 bytes of the kernels' 32-bit offsets: 1280 chunks, with 4-byte
+    pair loads at the even length and 16-bit ones at the odd. The inputs have a
+    closed form:
     delta = 0.5 (softplus off), A = -1, B = C = 1, no D, no gate, and
     u[c, t] = ((5 t + c) mod 9) - 4, so y[c, t] = 16 x_t of the recurrence in
     helpers.steady_scan_table, which after 200 steps (e^-100 of the start left) is
