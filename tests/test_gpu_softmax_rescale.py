@@ -182,3 +182,36 @@ def test_decode_fp8_climbing_scores(ops, splits):
     assert np.isfinite(got).all()
     assert max_abs(got, ref) <= TOL_FP8_ABS * max(1.0, np.abs(ref).max())
     assert max_abs(to_f32(lse), rl) <= TOL_LSE_ABS
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("B,Hk,L", [
+    (70, 8, 1024),   # 560 work-groups: one wave
+    (40, 8, 2048),   # 320: two waves (bf16; fp8 four, of which one holds half the ramp)
+    (2, 2, 4096),    # four
+], ids=["one_wave", "two_waves", "four_waves"])
+def test_decode_chains_climbing_scores(ops, B, Hk, L, fp8):
+    """One split, whose first wave's chain holds the whole ramp (1024 keys)."""
+    _log(f"case: decode chains climbing scores B={B} Hk={Hk} L={L} fp8={fp8}")
+    q = ramp_q((B, 4 * Hk, D), 11, torch.bfloat16)
+    k, v = (t.repeat(B, 1, 1, 1) for t in ramp_kv(1, Hk, L, 12, torch.bfloat16))
+    if fp8:
+        (kc, ks), (vc, vs) = (ops.kv_quantize_fp8(t.cuda()) for t in (k, v))
+        o, lse = ops.decode_splitk(q.cuda(), kc, vc, k_scale=ks, v_scale=vs, num_splits=1,
+                                   return_lse=True)
+    else:
+        o, lse = ops.decode_splitk(q.cuda(), k.cuda(), v.cuda(), num_splits=1, return_lse=True)
+    torch.cuda.synchronize()
+    for b in (0, B - 1):
+        one = slice(b, b + 1)
+        if fp8:
+            kv = [t[one].contiguous().cpu().numpy() for t in (kc, vc, ks, vs)]
+            ro, rl, _ = oracle.decode_splitk(bits(q[one]), kv[0], kv[1], oracle.FP8, kv[2], kv[3],
+                                             num_splits=1)
+        else:
+            ro, rl, _ = oracle.decode_splitk(bits(q[one]), bits(k[one]), bits(v[one]), oracle.BF16,
+                                             num_splits=1)
+        ref, got = oracle.decode(ro, oracle.BF16), to_f32(o[one])
+        assert np.isfinite(got).all()
+        assert max_abs(got, ref) <= (TOL_FP8_ABS if fp8 else TOL_BF16_ABS) * max(1.0, np.abs(ref).max())
+        assert max_abs(to_f32(lse[one]), rl) <= TOL_LSE_ABS
