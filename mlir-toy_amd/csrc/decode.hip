@@ -999,8 +999,8 @@ bool decode_supported(const DecodeLaunch &a, const char **why) {
 // (B1 L32768) 28.3 / 29.0 / 33.2; fp8, whose ring takes half the LDS, 512
 // 14.7 / 14.5 / 13.5, 1024 20.2 / 20.1 / 20.5.
 int decode_waves(int64_t groups, bool fp8) {
-  if (groups <= (fp8 ? 512 : 256)) return 4;
-  return groups <= 512 ? 2 : 1;
+  if (groups > 512) return 1;
+  return fp8 || groups <= 256 ? 4 : 2;
 }
 
 hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
@@ -1048,18 +1048,15 @@ hipError_t launch_decode(const DecodeLaunch &L, hipStream_t s) {
   a.scaled = paged && (L.chunk >= 512 || grid > 1280);
   a.sorted = paged && L.batch > 1 && L.batch <= 64 && L.chunk >= 512 && L.seq_kv < 1 << 25;
   const int rw = decode_waves(grid, L.kv_dtype == 3);
-  auto partial = [&](auto RW) {
-    constexpr int W = decltype(RW)::value;
-    auto k = L.kv_dtype == 3 ? (paged ? decode_partial_ring8<true, W> : decode_partial_ring8<false, W>)
-                             : (paged ? decode_partial_ring<true, W> : decode_partial_ring<false, W>);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(64 * W), 0, s, a);
-  };
-  if (rw == 4)
-    partial(std::integral_constant<int, 4>{});
-  else if (rw == 2)
-    partial(std::integral_constant<int, 2>{});
+  auto partial = [&](auto k) { hipLaunchKernelGGL(k, dim3(grid), dim3(64 * rw), 0, s, a); };
+  if (rw == 2)  // bf16
+    partial(paged ? decode_partial_ring<true, 2> : decode_partial_ring<false, 2>);
+  else if (L.kv_dtype == 3)
+    partial(rw == 4 ? (paged ? decode_partial_ring8<true, 4> : decode_partial_ring8<false, 4>)
+                    : (paged ? decode_partial_ring8<true, 1> : decode_partial_ring8<false, 1>));
   else
-    partial(std::integral_constant<int, 1>{});
+    partial(rw == 4 ? (paged ? decode_partial_ring<true, 4> : decode_partial_ring<false, 4>)
+                    : (paged ? decode_partial_ring<true, 1> : decode_partial_ring<false, 1>));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (L.splits == 1) return hipSuccess;
