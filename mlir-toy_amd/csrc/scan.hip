@@ -495,10 +495,10 @@ __global__ __launch_bounds__(NT, 5) void selective_scan_out(ScanArgs a) {
 // is and reach a finite state where 2^e alone is past fp32 (decays above 1: A
 // or delta of the other sign), so the same holds here.
 __device__ inline float advance(float e, float x, float c) {
-  if (x == 0.0f || __builtin_isinf(x)) return x + c;
   const bool far = e > 126.0f;
   const float f = fast_exp2(far ? 0.5f * e : e);
-  return fmaf(f, far ? f * x : x, c);
+  const float r = fmaf(f, far ? f * x : x, c);
+  return x == 0.0f || __builtin_isinf(x) ? x + c : r;
 }
 
 // The carry pass: one lane per (batch row, channel, state) walks the chunks
